@@ -1,0 +1,82 @@
+"""GPU tier: the streaming decode at head_dim 64 and 256 and in float32.
+
+The same partition logic as the 16-bit head_dim 128 kernel
+(test_gpu_decode_stream.py) over other row lengths: 128-byte rows (two to a
+LDS bank window, 8 rows a load), 512-byte rows (16-key stages) and float32
+products, at the edges of their stages and page groups, on grids that leave
+sequences whole, cut in a few pieces and cut in one piece per stage (each
+combine form). Oracle: flash_attention.py:555-589 decode on the cache prefix,
+paged.py:45-99 over the gathered pages.
+"""
+
+from __future__ import annotations
+
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import check_fwd, dev, host, note
+from oracle import decode_ref, paged_ref
+from pallas_flash import _lib, flash_attention_decode, paged_flash_attention
+
+pytestmark = pytest.mark.gpu
+
+FORMS = [("bf16", 64), ("f16", 64), ("bf16", 256), ("f16", 256), ("f32", 64), ("f32", 128)]
+
+
+def _waves(w):
+    return contextlib.nullcontext() if w is None else _lib.tuning(decode_waves=w)
+
+
+@pytest.mark.parametrize("w", [None, 1, 7])
+@pytest.mark.parametrize("dt,D", FORMS)
+@pytest.mark.parametrize("B,Hq,Hkv,cap,L", [
+    (3, 8, 2, 70, 1),       # one key; g = 4
+    (2, 10, 2, 64, 15),     # g = 5: 16 query rows, a short 16-key stage
+    (2, 32, 2, 64, 33),     # g = 16: every query row; one key past a stage
+    (1, 1, 1, 1300, 1299),  # one sequence cut in dozens of pieces
+    (2, 34, 2, 40, 17),     # g = 17: the generic kernel
+])
+def test_decode(w, dt, D, B, Hq, Hkv, cap, L):
+    note(f"stream decode waves={w} {dt} D={D} B={B} Hq={Hq} Hkv={Hkv} cap={cap} L={L}")
+    rng = np.random.default_rng(L)
+    q = rng.standard_normal((B, Hq, 1, D))
+    k, v = rng.standard_normal((2, B, Hkv, cap, D))
+    k[:, :, L:] = v[:, :, L:] = np.nan
+    tq, tk, tv = dev(q, dt), dev(k, dt), dev(v, dt)
+    with _waves(w):
+        out = host(flash_attention_decode(tq, tk, tv, L))
+    check_fwd(out, decode_ref(host(tq), host(tk), host(tv), L), dt)
+
+
+@pytest.mark.parametrize("w", [None, 5])
+@pytest.mark.parametrize("dt,D", FORMS)
+@pytest.mark.parametrize("page", [4, 8, 12, 16, 48, 64])
+def test_paged(w, dt, D, page):
+    note(f"stream paged waves={w} {dt} D={D} page={page}")
+    rng = np.random.default_rng(page)
+    B, Hq, Hkv, pps = 6, 8, 2, 20
+    lens = np.array([0, 1, 15, 33, 5 * page + 3, pps * page], np.int32)
+    used = -(-lens // page)
+    npages = int(used.sum()) + 3
+    perm = rng.permutation(npages)
+    table = np.full((B, pps), -1, np.int32)
+    cur = 0
+    for b, n in enumerate(used):
+        table[b, :n] = perm[cur:cur + n]
+        cur += n
+    q = rng.standard_normal((B, Hq, 1, D))
+    kp, vp = rng.standard_normal((2, npages, Hkv, page, D))
+    kp[perm[cur:]] = vp[perm[cur:]] = np.nan  # pages of no sequence
+    for b, n in enumerate(used):
+        if lens[b] % page:
+            kp[table[b, n - 1], :, lens[b] % page:] = np.nan
+            vp[table[b, n - 1], :, lens[b] % page:] = np.nan
+    tq, tk, tv = dev(q, dt), dev(kp, dt), dev(vp, dt)
+    with _waves(w):
+        out = host(paged_flash_attention(tq, tk, tv, torch.as_tensor(table), torch.as_tensor(lens)))
+    clean = lambda t: np.nan_to_num(host(t))
+    check_fwd(out, paged_ref(host(tq), clean(tk), clean(tv), np.where(table < 0, 0, table), lens), dt)
+    assert (out[0] == 0).all()

@@ -44,6 +44,8 @@ SOURCES = {
     "attn_bwd_f32.hip": [],
     "attn_bwd_d256.hip": [],
     "decode_stream.hip": [],
+    "decode_stream_dims.hip": [],
+    "decode_stream_f32.hip": [],
 }
 
 # sources whose MFMAs are (partly) inline assembly: the result-read check

@@ -335,22 +335,40 @@ static int decode_chunk(int64_t units, int max_len) {
   return (int)chunk;
 }
 
-// Streaming kernel (decode_stream.hip): a persistent grid of one-wave
+// Streaming kernel (decode_stream.hpp): a persistent grid of one-wave
 // workgroups, as many as are resident at once (queried once per device),
 // with an LDS ring of 2 stages (measured on MI355X: 2 stages x 4 waves per
-// CU beat 3 x 3 and 4 x 2). Tuning and test overrides: decode_stages (2..4)
-// and decode_waves (grid size; any value >= 1 is correct, only the resident
-// count is fast).
-static int stream_setup(pf::DecodeParams* p, int group) {
+// CU beat 3 x 3 and 4 x 2). Tuning and test overrides: decode_stages (2..4,
+// of the 16-bit head_dim 128 kernels) and decode_waves (grid size; any value
+// >= 1 is correct, only the resident count is fast).
+// A short problem starts only as many waves as it has stages (32 keys; 16 in
+// float32 at head_dim 128), and keeps no partial slots for more; at 16-bit
+// head_dim 256 a wave takes at least two 16-key stages, which halves the slots
+// for 0.6 us. One stage a wave also cuts equal sequences alike, whatever
+// their place in the list. max_len: the most keys a sequence can have.
+static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   Tuning& t = tuning();
   const int ns = t.decode_stages.load(std::memory_order_relaxed);
   p->stages = ns;
   const int wv = t.decode_waves.load(std::memory_order_relaxed);
-  p->n_waves = wv > 0 ? wv : pf::decode_stream_waves(ns, group);
+  const int group = p->Hq / p->Hkv;
+  p->n_waves = wv > 0 ? wv : pf::decode_stream_waves(dtype, p->D, ns, group);
+  const int unit = dtype == PF_DTYPE_F32 && p->D == 128 ? 16 : 32;
+  const int64_t runs = (int64_t)p->B * p->Hkv * ((group + 15) / 16) * ((max_len + unit - 1) / unit);
+  if (p->n_waves > runs) p->n_waves = (int)(runs > 1 ? runs : 1);
   p->n_split = 0;
   p->chunk = 0;
   return p->n_waves;
 }
+
+// Whether the streaming kernel's 32-bit byte offsets reach every row of a run
+// of `rows` rows (a cache slot range or a page).
+static bool stream_range_ok(int64_t rows, int32_t head_dim, int32_t dtype) {
+  return rows * head_dim * (dtype == PF_DTYPE_F32 ? 4 : 2) < ((int64_t)1 << 31);
+}
+// The 16-bit head_dim 128 forms run on the streaming kernel alone; the others
+// fall back to the generic kernel past its range.
+static bool stream_only(int32_t head_dim, int32_t dtype) { return head_dim == 128 && dtype != PF_DTYPE_F32; }
 
 static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   if (!a) return PF_ERR_INVALID;
@@ -376,11 +394,13 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   p->cache_size = a->cache_size;
   p->cache_len = a->cache_len;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
-  if (pf::decode_stream_supported(a->dtype, a->head_dim, false, 0)) {
+  if (pf::decode_stream_supported(a->dtype, a->head_dim, g, false, 0)) {
     // buffer offsets within one (b, kv head) run are 32-bit
-    if ((int64_t)a->cache_size * a->head_dim * 2 >= ((int64_t)1 << 31)) return PF_ERR_UNSUPPORTED;
-    if (stream_setup(p, g) <= 0) return PF_ERR_LAUNCH;
-    return PF_OK;
+    if (stream_range_ok(a->cache_size, a->head_dim, a->dtype)) {
+      if (stream_setup(p, a->dtype, a->cache_len) <= 0) return PF_ERR_LAUNCH;
+      return PF_OK;
+    }
+    if (stream_only(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
   }
   p->chunk = decode_chunk(units, a->cache_len);
   p->n_split = (a->cache_len + p->chunk - 1) / p->chunk;
@@ -388,10 +408,14 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   return PF_OK;
 }
 
-// Partial slots: streaming kernel 2 per wave x query rows; generic kernel
-// one per (b, query head, chunk).
+// Partial slots: streaming kernel one per piece (piece_slot) x query rows;
+// generic kernel one per (b, query head, chunk).
 static size_t decode_slots(const pf::DecodeParams& p) {
-  if (p.n_waves > 0) return (size_t)2 * p.n_waves * pf::decode_stream_qrows(p.Hq / p.Hkv);
+  if (p.n_waves > 0) {
+    const int group = p.Hq / p.Hkv;
+    const int64_t seqs = (int64_t)p.B * p.Hkv * ((group + 15) / 16);
+    return (size_t)(p.n_waves + (seqs < p.n_waves ? seqs : p.n_waves)) * pf::decode_stream_qrows(group);
+  }
   return (size_t)p.B * p.Hq * p.n_split;
 }
 
@@ -457,10 +481,12 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p) {
   p->page_size = a->page_size;
   p->pages_per_seq = a->pages_per_seq;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
-  if (pf::decode_stream_supported(a->dtype, a->head_dim, true, a->page_size)) {
-    if ((int64_t)a->page_size * a->head_dim * 2 >= ((int64_t)1 << 31)) return PF_ERR_UNSUPPORTED;
-    if (stream_setup(p, g) <= 0) return PF_ERR_LAUNCH;
-    return PF_OK;
+  if (pf::decode_stream_supported(a->dtype, a->head_dim, g, true, a->page_size)) {
+    if (stream_range_ok(a->page_size, a->head_dim, a->dtype)) {
+      if (stream_setup(p, a->dtype, max_len) <= 0) return PF_ERR_LAUNCH;
+      return PF_OK;
+    }
+    if (stream_only(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
   }
   p->chunk = decode_chunk(units, (int)(max_len > 0 ? max_len : 1));
   p->n_split = max_len > 0 ? (int)((max_len + p->chunk - 1) / p->chunk) : 1;
@@ -609,8 +635,8 @@ static int fill_decode_step(const pf_attn_decode_step_args* a, pf::DecodeParams*
   if (a->cos != nullptr && a->rope_len < 1) return PF_ERR_INVALID;
   if (!isfinite(a->sm_scale)) return PF_ERR_INVALID;
   if (!dtype_ok(a->dtype)) return PF_ERR_UNSUPPORTED;
-  if (!pf::decode_stream_supported(a->dtype, a->head_dim, false, 0)) return PF_ERR_UNSUPPORTED;
-  if ((int64_t)a->cache_size * a->head_dim * 2 >= ((int64_t)1 << 31)) return PF_ERR_UNSUPPORTED;
+  if (!stream_only(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;  // 16-bit head_dim 128
+  if (!stream_range_ok(a->cache_size, a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
   *p = pf::DecodeParams{};
   p->q = a->q;
   p->k = a->k_cache;
@@ -634,7 +660,7 @@ static int fill_decode_step(const pf_attn_decode_step_args* a, pf::DecodeParams*
   p->v_new = a->v_new;
   p->k_out = a->k_cache;
   p->v_out = a->v_cache;
-  if (stream_setup(p, a->num_heads / a->num_kv_heads) <= 0) return PF_ERR_LAUNCH;
+  if (stream_setup(p, a->dtype, a->cache_size) <= 0) return PF_ERR_LAUNCH;
   return PF_OK;
 }
 

@@ -361,9 +361,7 @@ hipError_t launch_decode_combine(const DecodeParams& p, int dtype, bool paged, h
 }
 
 hipError_t launch_decode(const DecodeParams& p, int dtype, bool paged, hipStream_t stream) {
-  // the streaming kernel reads rows of exactly its compute width
-  if (p.dr == p.D && decode_stream_supported(dtype, p.dr, paged, p.page_size))
-    return launch_decode_stream(p, dtype, paged, stream);
+  if (p.n_waves > 0) return launch_decode_stream(p, dtype, paged, stream);
   hipError_t e = paged ? launch_dtype<true>(p, dtype, false, stream) : launch_dtype<false>(p, dtype, false, stream);
   if (e != hipSuccess) return e;
   return launch_decode_combine(p, dtype, paged, stream);

@@ -195,7 +195,7 @@ struct DecodeParams {
   int chunk;          // keys per chunk (multiple of 32)
   float scale_log2;
   int stages;         // streaming kernel: LDS ring depth (2..4)
-  int n_waves;        // streaming kernel: persistent grid (one wave per workgroup)
+  int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
   // Fused decode step (streaming kernel, positions != null): the new token of
   // batch b is at pos = positions[b * pos_stride]; its k (rotated with table
   // row pos) and v go to cache slot pos (ring: pos % cache_size) and it
@@ -214,12 +214,15 @@ struct DecodeParams {
   void* v_out;
 };
 
-// Split-KV partials + combine; picks the streaming kernel (decode_stream.hip)
-// when decode_stream_supported() holds, else the generic one (decode.hip).
+// Split-KV partials + combine: the streaming kernel (decode_stream.hpp) when
+// the caller planned a persistent grid for it (n_waves > 0, only where
+// decode_stream_supported() holds), else the generic one (decode.hip).
 hipError_t launch_decode(const DecodeParams& p, int dtype, bool paged, hipStream_t stream);
 hipError_t launch_decode_combine(const DecodeParams& p, int dtype, bool paged, hipStream_t stream);
-bool decode_stream_supported(int dtype, int head_dim, bool paged, int page_size);
-int decode_stream_waves(int stages, int group);  // resident one-wave workgroups on this device
+// group: query heads per kv head
+bool decode_stream_supported(int dtype, int head_dim, int group, bool paged, int page_size);
+// resident one-wave workgroups on this device
+int decode_stream_waves(int dtype, int head_dim, int stages, int group);
 int decode_stream_qrows(int group);               // query rows per partial slot
 hipError_t launch_decode_stream(const DecodeParams& p, int dtype, bool paged, hipStream_t stream);
 
