@@ -93,6 +93,16 @@ typedef struct {
 
 int pf_attn_fwd(const pf_attn_fwd_args* args, void* stream);
 
+/* The forward with a workspace: a call with fewer work items than the GPU has
+ * CUs (a short prompt, few heads, a few queries against many keys) cuts its
+ * key range into chunks that run side by side and leave float32 partials in
+ * `workspace`, which a second kernel merges; the results equal pf_attn_fwd's
+ * to float32 rounding. pf_attn_fwd_workspace_size(args) bytes (0: this call
+ * gains nothing from it, and workspace may be NULL), 256-byte aligned device
+ * memory, contents on entry do not matter. A smaller one: PF_ERR_WORKSPACE. */
+size_t pf_attn_fwd_workspace_size(const pf_attn_fwd_args* args);
+int pf_attn_fwd_ws(const pf_attn_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Fused-RoPE forward (no LSE). Replaces the `flash_attention_rope_fwd`
  * pallas_call (fused_rope.py:183-213, kernel :53-113). Rotation is
@@ -106,7 +116,10 @@ int pf_attn_fwd(const pf_attn_fwd_args* args, void* stream);
  *   q_cos, q_sin [seq_len_q, head_dim] float32
  *   k_cos, k_sin [seq_len_k, head_dim] float32
  *   workspace: at least pf_attn_fwd_rope_workspace_size(args) bytes,
- *              256-byte aligned device memory (contents on entry do not matter)
+ *              256-byte aligned device memory (contents on entry do not matter);
+ *              the rotated K, and the partials of a split key range as in
+ *              pf_attn_fwd_ws (a workspace of K's size alone, rounded up to
+ *              256 bytes, runs without the split)
  * Other fields as pf_attn_fwd_args (lse is ignored and may be NULL).
  * ------------------------------------------------------------------------- */
 typedef struct {
@@ -190,6 +203,11 @@ int pf_attn_bwd_dq(const pf_attn_bwd_args* args, void* stream);
 int pf_attn_bwd_dkv(const pf_attn_bwd_args* args, void* stream);
 /* dq (which also writes delta), then dkv, on one stream */
 int pf_attn_bwd(const pf_attn_bwd_args* args, void* stream);
+/* pf_attn_bwd with a workspace (as pf_attn_fwd_ws): with few work items dQ runs
+ * by chunks of keys and dK/dV by runs of query blocks, and a third kernel sums
+ * their float32 partials. */
+size_t pf_attn_bwd_workspace_size(const pf_attn_bwd_args* args);
+int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Single-query decode against a contiguous KV cache. Replaces

@@ -8,10 +8,11 @@
 namespace pf {
 
 hipError_t launch_bwd_delta_f32(const BwdParams& p, int head_dim, hipStream_t stream);
+hipError_t launch_bwd_reduce_f32(const BwdParams& p, int head_dim, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int head_dim, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dkv_f32(const BwdParams& p, int head_dim, bool causal, hipStream_t stream);
 hipError_t launch_bwd_dkv16(const BwdParams& p, int dtype, int head_dim, bool causal, hipStream_t stream);
-// kernel 0 = delta, 1 = dQ, 2 = dK/dV
+// kernel 0 = delta, 1 = dQ, 2 = dK/dV, 3 = reduce
 hipError_t launch_bwd_d256(int kernel, const BwdParams& p, int dtype, bool causal, hipStream_t stream);
 
 #define PF_DISPATCH16(FN, ...)                                                 \
@@ -30,6 +31,12 @@ hipError_t launch_attn_bwd_delta(const BwdParams& p, int dtype, int head_dim, hi
   if (dtype == kF32) return launch_bwd_delta_f32(p, head_dim, stream);
   if (head_dim == 256) return launch_bwd_d256(0, p, dtype, false, stream);
   PF_DISPATCH16(delta_typed, p, stream);
+}
+
+hipError_t launch_attn_bwd_reduce(const BwdParams& p, int dtype, int head_dim, bool causal, hipStream_t stream) {
+  if (dtype == kF32) return launch_bwd_reduce_f32(p, head_dim, causal, stream);
+  if (head_dim == 256) return launch_bwd_d256(3, p, dtype, causal, stream);
+  PF_DISPATCH16(reduce_typed, p, causal, stream);
 }
 
 hipError_t launch_attn_bwd_dq(const BwdParams& p, int dtype, int head_dim, bool causal,

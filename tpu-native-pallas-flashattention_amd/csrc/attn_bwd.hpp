@@ -33,6 +33,7 @@
 #include "pf_kernels.hpp"
 #include "pf_tiles.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace pf {
@@ -65,7 +66,10 @@ __global__ __launch_bounds__(256) void pf_attn_bwd_delta_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool CAUSAL>
+// SPLIT: a workgroup per chunk of chunk_q keys (a multiple of 64); K/V bases, kv_len and the causal limit move by the chunk's
+// first key. The chunks' float32 sums go to part_dq and are added by
+// pf_attn_bwd_reduce_kernel, unless the item needs one chunk only.
+template <typename T, int D, bool CAUSAL, bool SPLIT = false>
 __global__ __launch_bounds__(256, (kWgPerCu<T, D>))
 void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   using MF = Mfma32<T>;
@@ -80,9 +84,18 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   __shared__ __attribute__((aligned(16))) char smem[4 * G::BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, hh = lane >> 5, l32 = lane & 31;
-  const int item = work_tail_item(p.tail, n_work, reinterpret_cast<int*>(smem));
-  if (item < 0) return;
-  const int w = xcd_remap(item, n_work, p.g);
+  int w;  // (query block from the last one down, batch, kv head, group member)
+  [[maybe_unused]] int split = 0;
+  if constexpr (SPLIT) {
+    const SplitItem it = split_item(blockIdx.x, n_qblk, p.B * p.Hq,
+                                    [&](int i) { return dq_chunks<CAUSAL>(p, (n_qblk - 1 - i) * 128); });
+    w = it.blk * p.B * p.Hq + it.member;
+    split = it.chunk;
+  } else {
+    const int item = work_tail_item(p.tail, n_work, reinterpret_cast<int*>(smem));
+    if (item < 0) return;
+    w = xcd_remap(item, n_work, p.g);
+  }
   const int member = w % p.g;
   int rest = w / p.g;
   const int kvh = rest % p.Hkv;
@@ -101,6 +114,15 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   const T* dOb = static_cast<const T*>(p.dout) + qoff * D;
   const T* Kb = static_cast<const T*>(p.k) + (int64_t)(b * p.Hkv + kvh) * p.Sk * D;
   const T* Vb = static_cast<const T*>(p.v) + (int64_t)(b * p.Hkv + kvh) * p.Sk * D;
+  [[maybe_unused]] int kc0 = 0, n_chunk = 1;
+  int kv_len = p.kv_len;
+  if constexpr (SPLIT) {
+    n_chunk = dq_chunks<CAUSAL>(p, q0);
+    kc0 = split * p.chunk_q;
+    kv_len = min(kv_len - kc0, p.chunk_q);
+    Kb += (int64_t)kc0 * D;
+    Vb += (int64_t)kc0 * D;
+  }
 
   Frag qf[QF], dof[QF];
   load_row_frags<T, D>(Qb, qrow, qvalid, hh, qf);
@@ -129,14 +151,14 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
       for (int e = 0; e < EPC; ++e) part += a[e] * d[e];
     }
     dlt = qvalid ? wave_xor32_sum(part) : 0.f;
-    if (qvalid && hh == 0) p.delta[qoff + qrow] = dlt;
+    if (qvalid && hh == 0 && (!SPLIT || split == 0)) p.delta[qoff + qrow] = dlt;
   }
 
   f32x16 acc[NDT];
 #pragma unroll
   for (int i = 0; i < NDT; ++i) acc[i] = (f32x16)(0.f);
 
-  const uint32_t kv_bytes = (uint32_t)p.kv_len * (uint32_t)G::RB;
+  const uint32_t kv_bytes = (uint32_t)kv_len * (uint32_t)G::RB;
   const i32x4 krs = make_desc(Kb, kv_bytes);
   const i32x4 vrs = make_desc(Vb, kv_bytes);
   TileDma<T, D> dma;
@@ -144,8 +166,8 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   TrAddr<T, D> kta;
   kta.init(lane);
 
-  int kv_end = p.kv_len;
-  if constexpr (CAUSAL) kv_end = min(kv_end, min(q0 + BM, p.Sq));
+  int kv_end = kv_len;
+  if constexpr (CAUSAL) kv_end = min(kv_end, min(q0 + BM, p.Sq) - kc0);
   const int nblk = (kv_end + BN - 1) / BN;
 
   if (nblk > 0) {
@@ -160,11 +182,11 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   // all rows inside Sq), then the rest (diagonal, kv_len tail) with the mask.
   // Every wave runs every block: one whose keys are all masked for its rows
   // adds exact zeros (dS = 0).
-  int n_plain = (q0 + BM > p.Sq) ? 0 : min(nblk, p.kv_len / BN);
-  if constexpr (CAUSAL) n_plain = min(n_plain, q0 / BN);
+  int n_plain = (q0 + BM > p.Sq) ? 0 : min(nblk, kv_len / BN);
+  if constexpr (CAUSAL) n_plain = min(n_plain, max(0, q0 - kc0) / BN);  // a chunk may start past q0
 
   // Valid keys of this lane's query: key < klim (kv_len, and causal key <= q).
-  const int klim = qvalid ? (CAUSAL ? min(p.kv_len, qrow + 1) : p.kv_len) : 0;
+  const int klim = qvalid ? (CAUSAL ? min(kv_len, qrow + 1 - kc0) : kv_len) : 0;
   auto block = [&](auto masked, int j) {
     const int kv0 = j * BN;
     // masked blocks: bit 16t + r says whether key kv0 + 32hh + 16t + r is valid
@@ -303,6 +325,13 @@ void pf_attn_bwd_dq_kernel(BwdParams p, int n_qblk, int n_work) {
   for (int j = 0; j < n_plain; ++j) block(std::false_type{}, j);
   for (int j = n_plain; j < nblk; ++j) block(std::true_type{}, j);
 
+  if constexpr (SPLIT) {
+    if (n_chunk > 1) {
+      const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+      if (qvalid) store_acc_row<float, D>(p.part_dq + (split * rows + qoff + qrow) * D, acc, 1.f, hh);
+      return;
+    }
+  }
   if (qvalid) store_acc_row<T, D>(static_cast<T*>(p.dq) + (qoff + qrow) * D, acc, p.sm_scale, hh);
 }
 
@@ -331,7 +360,10 @@ __host__ __device__ constexpr int dkv_phase0_op(int k, int n, int dly) {
   }
   return 0;
 }
-template <typename T, int D, bool CAUSAL>
+// SPLIT: a workgroup per run of steps_k steps of the loop below (its order unchanged); the runs' float32 sums go to part_dk and
+// part_dv and are added by pf_attn_bwd_reduce_kernel, unless the item needs one
+// run only.
+template <typename T, int D, bool CAUSAL, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, int n_kblk) {
   using MF = Mfma32<T>;
   using Frag = typename MF::Frag;
@@ -344,7 +376,8 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
   // (whose 128-row double buffer would exceed the LDS and whose dK/dV
   // accumulators alone fill the AGPRs): 64 rows with the plain step body.
   constexpr bool kAcc = sizeof(T) == 2 && D <= 128;
-  constexpr int BNK = 128, BMQ = kAcc ? 128 : 64, NSUB = BMQ / 64;
+  constexpr int BNK = 128, BMQ = kDkvRows<T, D>, NSUB = BMQ / 64;
+  static_assert(!kAcc || BMQ == 128, "the fenced sequence runs two 64-row passes");
   constexpr int KF = (D / 2) / MF::kK;
   constexpr int NDT = D / 32;
   constexpr int PF = 32 / MF::kK;
@@ -364,7 +397,14 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, hh = lane >> 5, l32 = lane & 31;
   // heavy first: for causal, early key blocks are attended by the most queries
-  const int w = blockIdx.x;
+  int w = blockIdx.x;
+  [[maybe_unused]] int split = 0;
+  if constexpr (SPLIT) {
+    const SplitItem it = split_item(blockIdx.x, n_kblk, p.B * p.Hkv,
+                                    [&](int i) { return dkv_runs(p, 128 * i, BMQ, CAUSAL); });
+    w = it.blk * p.B * p.Hkv + it.member;
+    split = it.chunk;
+  }
   const int kblk = w / (p.B * p.Hkv);
   const int bk = w % (p.B * p.Hkv);
   const int b = bk / p.Hkv, kvh = bk % p.Hkv;
@@ -373,6 +413,13 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
   const int wk0 = k0 + 32 * wv;
   const int kkey = wk0 + l32;
   const bool kvalid = kkey < p.kv_len;
+
+  int st_begin = 0;  // this run's first step
+  [[maybe_unused]] int n_run = 1;
+  if constexpr (SPLIT) {
+    n_run = dkv_runs(p, k0, BMQ, CAUSAL);
+    st_begin = split * p.steps_k;
+  }
 
   const int64_t koff = (int64_t)(b * p.Hkv + kvh) * p.Sk;
   Frag kf[KF], vf[KF];
@@ -388,7 +435,7 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
 
   const int q_begin = CAUSAL ? (k0 / BMQ) * BMQ : 0;
   const int nqb = (k0 < p.kv_len && q_begin < p.Sq) ? (p.Sq - q_begin + BMQ - 1) / BMQ : 0;
-  const int nsteps = nqb * p.g;  // (group member, q block) pairs
+  int nsteps = nqb * p.g;  // (group member, q block) pairs
 
   // Step order: every step that needs a mask for some wave of the workgroup
   // first, then the rest (order below), so each of the two loops has one straight-
@@ -473,11 +520,17 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
   };
 
   Pos pos{0, 0};  // of step 0 (a masked or an unmasked step alike)
-  if (nsteps > 0) {
+  if constexpr (SPLIT) {
+    nsteps = min(nsteps, st_begin + p.steps_k);
+    if (st_begin < n_masked) pos = Pos{st_begin / m_pm, st_begin % m_pm};
+    else pos = Pos{(st_begin - n_masked) % p.g, (st_begin - n_masked) / p.g};
+  }
+  if (st_begin < nsteps) {
     int h0, qb00;
-    coords(0, pos, h0, qb00);
-    load_step(h0, qb00, smem);
-    store_step(smem, qb00);
+    coords(st_begin, pos, h0, qb00);
+    char* const buf0 = smem + (st_begin & 1) * BUF;
+    load_step(h0, qb00, buf0);
+    store_step(buf0, qb00);
   }
   dma_wait();
   __syncthreads();
@@ -740,7 +793,7 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
     }
   };
 
-  int st = 0;
+  int st = st_begin;
   auto run = [&](auto masked, int st_end) {
     for (; st < st_end; ++st) {
       const char* buf = smem + (st & 1) * BUF;
@@ -765,7 +818,7 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
       __syncthreads();
     }
   };
-  run(std::true_type{}, n_masked);
+  run(std::true_type{}, SPLIT ? min(n_masked, nsteps) : n_masked);
   run(std::false_type{}, nsteps);
 
   if constexpr (kAcc) {
@@ -775,10 +828,66 @@ __global__ __launch_bounds__(256, 1) void pf_attn_bwd_dkv_kernel(BwdParams p, in
       agpr_fence(dv[i]);
     }
   }
+  if constexpr (SPLIT) {
+    if (n_run > 1) {
+      const int64_t row = (int64_t)split * p.B * p.Hkv * p.Sk + koff + kkey;
+      if (kkey < p.Sk) {
+        store_acc_row<float, DA>(p.part_dk + row * D + dcol, dk, 1.f, hh);
+        store_acc_row<float, DA>(p.part_dv + row * D + dcol, dv, 1.f, hh);
+      }
+      return;
+    }
+  }
   if (kkey < p.Sk) {
     store_acc_row<T, DA>(static_cast<T*>(p.dk) + (koff + kkey) * D + dcol, dk, p.sm_scale, hh);
     store_acc_row<T, DA>(static_cast<T*>(p.dv) + (koff + kkey) * D + dcol, dv, 1.f, hh);
   }
+}
+
+// Sum the partials of split dQ items (blockIdx.y == 0) and split dK/dV items
+// (1, 2), scale and round once. D / 4 lanes per row, 16 bytes a lane. Rows whose
+// item needed one chunk or run were written by their kernel.
+template <typename T, int D, bool CAUSAL>
+__global__ __launch_bounds__(256) void pf_attn_bwd_reduce_kernel(BwdParams p) {
+  constexpr int LPR = D / 4, RPB = 256 / LPR, NB = 4;
+  const int which = blockIdx.y;
+  const int S = which == 0 ? p.Sq : p.Sk;
+  const int64_t rows = (int64_t)p.B * (which == 0 ? p.Hq : p.Hkv) * S;
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  const int sub = threadIdx.x % LPR;
+  if (row >= rows) return;
+  const int pos = (int)(row % S), start = pos & ~127;
+  int n;
+  if (which == 0) n = p.n_split_q > 1 ? dq_chunks<CAUSAL>(p, start) : 1;
+  else n = p.n_split_k > 1 ? dkv_runs(p, start, kDkvRows<T, D>, CAUSAL) : 1;
+  if (n <= 1) return;
+  const float* part = (which == 0 ? p.part_dq : which == 1 ? p.part_dk : p.part_dv) + row * D + 4 * sub;
+  f32x4 acc = (f32x4)(0.f);
+  for (int c0 = 0; c0 < n; c0 += NB) {
+    f32x4 v[NB];
+#pragma unroll
+    for (int c = 0; c < NB; ++c) v[c] = *reinterpret_cast<const f32x4*>(part + min(c0 + c, n - 1) * rows * D);
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+      if (c0 + c < n) acc += v[c];
+  }
+  const float mul = which == 2 ? 1.f : p.sm_scale;
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  v4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = Elem<T>::from_f32(acc[e] * mul);
+  *reinterpret_cast<v4*>(static_cast<T*>(which == 0 ? p.dq : which == 1 ? p.dk : p.dv) + row * D + 4 * sub) = y;
+}
+
+template <typename T, int D>
+hipError_t reduce_typed(const BwdParams& p, bool causal, hipStream_t st) {
+  constexpr int RPB = 256 / (D / 4);
+  int64_t rows = p.n_split_q > 1 ? (int64_t)p.B * p.Hq * p.Sq : 0;
+  if (p.n_split_k > 1) rows = std::max(rows, (int64_t)p.B * p.Hkv * p.Sk);
+  const dim3 grid((unsigned)((rows + RPB - 1) / RPB), p.n_split_k > 1 ? 3 : 1);
+  if (causal) hipLaunchKernelGGL((pf_attn_bwd_reduce_kernel<T, D, true>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((pf_attn_bwd_reduce_kernel<T, D, false>), grid, dim3(256), 0, st, p);
+  return hipGetLastError();
 }
 
 template <typename T, int D>
@@ -795,6 +904,14 @@ template <typename T, int D>
 hipError_t dq_typed(const BwdParams& p, bool causal, hipStream_t st) {
   const int n_qblk = (p.Sq + 127) / 128;
   const int n_work = bwd_dq_items(p);
+  if (p.n_split_q > 1) {
+    const dim3 sgrid((unsigned)p.grid_q);
+    if (causal)
+      hipLaunchKernelGGL((pf_attn_bwd_dq_kernel<T, D, true, true>), sgrid, dim3(256), 0, st, p, n_qblk, n_work);
+    else
+      hipLaunchKernelGGL((pf_attn_bwd_dq_kernel<T, D, false, true>), sgrid, dim3(256), 0, st, p, n_qblk, n_work);
+    return hipGetLastError();
+  }
   const dim3 grid(work_tail_grid(p.tail, n_work));
   if (causal)
     hipLaunchKernelGGL((pf_attn_bwd_dq_kernel<T, D, true>), grid, dim3(256), 0, st, p, n_qblk, n_work);
@@ -807,7 +924,16 @@ template <typename T, int D>
 hipError_t dkv_typed(const BwdParams& p, bool causal, hipStream_t st) {
   const int n_kblk = (p.Sk + 127) / 128;
   // head_dim 256: two workgroups per key block, one per 128-column half of dK/dV
-  const dim3 grid(bwd_dkv_items(p), D > 128 ? 2 : 1);
+  const int halves = D > 128 ? 2 : 1;
+  if (p.n_split_k > 1) {
+    const dim3 sgrid((unsigned)p.grid_k, halves);
+    if (causal)
+      hipLaunchKernelGGL((pf_attn_bwd_dkv_kernel<T, D, true, true>), sgrid, dim3(256), 0, st, p, n_kblk);
+    else
+      hipLaunchKernelGGL((pf_attn_bwd_dkv_kernel<T, D, false, true>), sgrid, dim3(256), 0, st, p, n_kblk);
+    return hipGetLastError();
+  }
+  const dim3 grid(bwd_dkv_items(p), halves);
   if (causal)
     hipLaunchKernelGGL((pf_attn_bwd_dkv_kernel<T, D, true>), grid, dim3(256), 0, st, p, n_kblk);
   else

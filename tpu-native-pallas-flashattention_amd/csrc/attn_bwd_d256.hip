@@ -15,6 +15,8 @@ hipError_t launch_bwd_d256(int kernel, const BwdParams& p, int dtype, bool causa
     case 1: return bf ? bwd::dq_typed<bf16_t, 256>(p, causal, stream) : bwd::dq_typed<f16_t, 256>(p, causal, stream);
     case 2:
       return bf ? bwd::dkv_typed<bf16_t, 256>(p, causal, stream) : bwd::dkv_typed<f16_t, 256>(p, causal, stream);
+    case 3:
+      return bf ? bwd::reduce_typed<bf16_t, 256>(p, causal, stream) : bwd::reduce_typed<f16_t, 256>(p, causal, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -12,6 +12,12 @@ hipError_t launch_bwd_delta_f32(const BwdParams& p, int head_dim, hipStream_t st
   return hipErrorInvalidValue;
 }
 
+hipError_t launch_bwd_reduce_f32(const BwdParams& p, int head_dim, bool causal, hipStream_t stream) {
+  if (head_dim == 128) return bwd::reduce_typed<float, 128>(p, causal, stream);
+  if (head_dim == 64) return bwd::reduce_typed<float, 64>(p, causal, stream);
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int head_dim, bool causal, hipStream_t stream) {
   if (head_dim == 128) return bwd::dq_typed<float, 128>(p, causal, stream);
   if (head_dim == 64) return bwd::dq_typed<float, 64>(p, causal, stream);

@@ -50,7 +50,15 @@ namespace {
 constexpr int kFwdBN = 64;   // keys per block
 
 
-template <typename T, int D, bool CAUSAL, bool ROPE>
+// SPLIT: a workgroup takes one chunk of p.chunk keys of its work item (causal:
+// p.chunk is a multiple of rpw, so a query block's rows all see the first key of
+// every chunk the block reaches). Everything below then runs on the chunk as if
+// it were the whole key range: K/V bases, kv_len and the causal limit move by
+// the chunk's first key. A block that needs one chunk only is finished here, the
+// others leave (max, sum, acc) for pf_attn_fwd_combine_kernel. Float32, 8 heads
+// of 512 rows and keys at head_dim 128: 32 whole items ran 73 us on 32 of 256
+// CUs.
+template <typename T, int D, bool CAUSAL, bool ROPE, bool SPLIT = false>
 __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdParams p) {
   using MF = Mfma32<T>;
   using Frag = typename MF::Frag;
@@ -88,9 +96,22 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
   // work item = (batch, kv head, head group, query block); the workgroup's
   // waves split into hpw heads x (4 / hpw) 32-row slices.
   int b, kvh, hg, qblk;
-  const int item = work_tail_item(p.tail, p.n_work, reinterpret_cast<int*>(smem));
-  if (item < 0) return;
-  fwd_work_item(item, p, b, kvh, hg, qblk);
+  [[maybe_unused]] int split = 0;
+  if constexpr (SPLIT) {
+    const int n_hg = p.g / p.hpw;
+    const SplitItem it =
+        split_item(blockIdx.x, p.n_qblk, p.B * p.Hkv * n_hg,
+                   [&](int i) { return fwd_chunks<CAUSAL>(p, (p.n_qblk - 1 - i) * p.rpw); });
+    qblk = p.n_qblk - 1 - it.blk;
+    hg = it.member % n_hg;
+    kvh = it.member / n_hg % p.Hkv;
+    b = it.member / (n_hg * p.Hkv);
+    split = it.chunk;
+  } else {
+    const int item = work_tail_item(p.tail, p.n_work, reinterpret_cast<int*>(smem));
+    if (item < 0) return;
+    fwd_work_item(item, p, b, kvh, hg, qblk);
+  }
   const int wph = 4 / p.hpw;  // waves per head
   const int h = kvh * p.g + hg * p.hpw + wv / wph;
 
@@ -101,17 +122,28 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
   const T* Qb = static_cast<const T*>(p.q) + (int64_t)(b * p.Hq + h) * p.Sq * D;
   const T* Kb = static_cast<const T*>(p.k) + (int64_t)(b * p.Hkv + kvh) * p.Sk * D;
   const T* Vb = static_cast<const T*>(p.v) + (int64_t)(b * p.Hkv + kvh) * p.Sk * D;
+  // Split: kc0 = the chunk's first key, n_chunk = the chunks of this query
+  // block; kv_len and the query positions the masks see are relative to kc0.
+  [[maybe_unused]] int kc0 = 0, n_chunk = 1;
+  int kv_len = p.kv_len;
+  if constexpr (SPLIT) {
+    n_chunk = fwd_chunks<CAUSAL>(p, q0);
+    kc0 = split * p.chunk;
+    kv_len = min(kv_len - kc0, p.chunk);
+    Kb += (int64_t)kc0 * D;
+    Vb += (int64_t)kc0 * D;
+  }
 
   // ---- staging: K/V rows at or past kv_len lie outside the buffer resources
   // and load as zeros (never read from memory). K and V go global -> LDS by
   // DMA (with fused RoPE, p.k is the K rotated once by pf_rope_rotate_k_kernel).
-  const uint32_t kv_bytes = (uint32_t)p.kv_len * (uint32_t)(D * ES);
+  const uint32_t kv_bytes = (uint32_t)kv_len * (uint32_t)(D * ES);
   const i32x4 krs = make_desc(Kb, kv_bytes);
   const i32x4 vrs = make_desc(Vb, kv_bytes);
   TileDma<T, D> dma;
   dma.init(tid);
-  int kv_end = p.kv_len;
-  if constexpr (CAUSAL) kv_end = min(kv_end, min(q0 + p.rpw, p.Sq));
+  int kv_end = kv_len;
+  if constexpr (CAUSAL) kv_end = min(kv_end, min(q0 + p.rpw, p.Sq) - kc0);
   const int nblk = (kv_end + BN - 1) / BN;
   // LDS: K tiles at [0, 2 BYTES) (block j in j & 1), V tiles after them.
   auto first_tiles = [&]() {
@@ -237,7 +269,9 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
   }
 
 
-  float m_run = kNegInf;  // running max, log2 domain (identical in both halves)
+  // Running max, log2 domain (identical in both halves). Split: a chunk whose
+  // scores are all -inf must leave an empty partial (sum 0), not exp2(-inf + inf).
+  float m_run = SPLIT ? -__FLT_MAX__ : kNegInf;
   float l_run = 0.f;      // running sum over this lane half's keys
   f32x16 acc[NDT];
 #pragma unroll
@@ -248,7 +282,7 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
   // the valid V rows up to a ~1e-30 relative perturbation of the weights).
   const float c2 = fmaxf(fabsf(p.scale_log2), 1e-30f);
   // Valid keys of this lane's query: key < lim (kv_len, and causal key <= q).
-  const int lim = CAUSAL ? min(p.kv_len, qrow + 1) : p.kv_len;
+  const int lim = CAUSAL ? min(kv_len, qrow + 1 - kc0) : kv_len;
 
   TrAddr<T, D> vta;
   vta.init(lane);
@@ -324,8 +358,8 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
   // Iteration j masks block j + 1. Blocks [0, n_plain) need no mask for any
   // row of the workgroup (below the causal diagonal, inside kv_len), so the
   // iterations run in two straight-line loops: plain max, then masked max.
-  int n_plain = min(nblk, p.kv_len / BN);
-  if constexpr (CAUSAL) n_plain = min(n_plain, (q0 + 1) / BN);
+  int n_plain = min(nblk, kv_len / BN);
+  if constexpr (CAUSAL) n_plain = min(n_plain, (q0 - kc0 + 1) / BN);
 
   // par = j & 1 as a compile-time constant: the LDS buffer addresses of an
   // iteration are then fixed and fold into the read instructions' offsets.
@@ -471,6 +505,16 @@ __global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdP
 
   // ---- finalize: o = acc / l, lse = m ln2 + ln l ---------------------------
   const float l_tot = wave_xor32_sum(l_run);
+  if constexpr (SPLIT) {
+    if (n_chunk > 1) {
+      if (qrow < p.Sq) {
+        const int64_t row = ((int64_t)split * p.B * p.Hq + (b * p.Hq + h)) * p.Sq + qrow;
+        store_acc_row<float, D>(p.part_o + row * D, acc, 1.f, hh);
+        if (hh == 0) *reinterpret_cast<f32x2*>(p.part_ml + 2 * row) = (f32x2){m_run, l_tot};
+      }
+      return;
+    }
+  }
   if (qrow < p.Sq) {
     // one correctly rounded reciprocal, then multiplies (within 1.5 ulp of
     // acc / l, instead of 64 full divisions per lane)
@@ -573,8 +617,70 @@ __global__ __launch_bounds__(256) void pf_rope_rotate_k_kernel(const T* __restri
   }
 }
 
+// Merge the chunks of the query blocks that needed more than one: o = sum_c
+// acc_c 2^(m_c - M) / sum_c l_c 2^(m_c - M), lse = M ln2 + ln(sum). D / 4 lanes
+// per row, 16 bytes a lane; every chunk of a row holds a valid key. Bound by
+// reading the partials back (and by its launch: 4-5 us at the sizes that
+// split).
+template <typename T, int D, bool CAUSAL>
+__global__ __launch_bounds__(256) void pf_attn_fwd_combine_kernel(FwdParams p) {
+  constexpr int LPR = D / 4, RPB = 256 / LPR, NB = 4;
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  const int sub = threadIdx.x % LPR;
+  if (row >= rows) return;
+  const int qrow = (int)(row % p.Sq);
+  const int n = fwd_chunks<CAUSAL>(p, qrow - qrow % p.rpw);
+  if (n <= 1) return;
+  float M = kNegInf;
+  for (int c = 0; c < n; ++c) M = fmaxf(M, p.part_ml[2 * (c * rows + row)]);
+  float l = 0.f;
+  f32x4 acc = (f32x4)(0.f);
+  for (int c0 = 0; c0 < n; c0 += NB) {
+    f32x4 v[NB];
+    f32x2 ml[NB];
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      const int64_t r = min(c0 + c, n - 1) * rows + row;
+      v[c] = *reinterpret_cast<const f32x4*>(p.part_o + r * D + 4 * sub);
+      ml[c] = *reinterpret_cast<const f32x2*>(p.part_ml + 2 * r);
+    }
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      if (c0 + c < n) {
+        const float w = __builtin_amdgcn_exp2f(ml[c][0] - M);
+        l += ml[c][1] * w;
+        acc += v[c] * w;
+      }
+    }
+  }
+  const float inv = 1.f / ((l == 0.f) ? 1.f : l);
+  T* out = static_cast<T*>(p.o) + row * D + 4 * sub;
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  v4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = Elem<T>::from_f32(acc[e] * inv);
+  *reinterpret_cast<v4*>(out) = y;
+  if (sub == 0 && p.lse != nullptr) p.lse[row] = (l == 0.f) ? 0.f : M * kLn2 + logf(l);
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_split(const FwdParams& p, bool rope, hipStream_t st) {
+  const dim3 grid((unsigned)p.split_grid), block(256);
+  if (rope) hipLaunchKernelGGL((pf_attn_fwd_kernel<T, D, CAUSAL, true, true>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((pf_attn_fwd_kernel<T, D, CAUSAL, false, true>), grid, block, 0, st, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  constexpr int RPB = 256 / (D / 4);
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
+  hipLaunchKernelGGL((pf_attn_fwd_combine_kernel<T, D, CAUSAL>), dim3((unsigned)((rows + RPB - 1) / RPB)), block, 0,
+                     st, p);
+  return hipGetLastError();
+}
+
 template <typename T, int D>
 hipError_t launch_typed(const FwdParams& p, bool causal, bool rope, hipStream_t st) {
+  if (p.n_split > 1) return causal ? launch_split<T, D, true>(p, rope, st) : launch_split<T, D, false>(p, rope, st);
   const dim3 grid(work_tail_grid(p.tail, p.n_work)), block(256);
   if (causal) {
     if (rope) hipLaunchKernelGGL((pf_attn_fwd_kernel<T, D, true, true>), grid, block, 0, st, p);

@@ -126,6 +126,9 @@ int fill_fwd(const pf_attn_fwd_args* a, pf::FwdParams* p) {
   p->n_work = (int)n_work;
   p->pair_group = fwd_pair_group(a);
   p->tail = pf::WorkTail{nullptr, p->n_work, 0};
+  p->n_split = 1;
+  p->chunk = p->split_grid = 0;
+  p->part_o = p->part_ml = nullptr;
   return PF_OK;
 }
 
@@ -155,6 +158,114 @@ pf::WorkTail plan_tail(int n_work, int min_items, hipStream_t stream) {
   w.n_static = n_static;
   w.n_tickets = (int)(pool * kTailSlack) + 1;
   return w;
+}
+
+// ---------------------------------------------------------------------------
+// Split plans. A prefill launch with fewer work items than CUs leaves CUs idle
+// while each item walks its whole key range (forward, dQ) or all its query
+// blocks (dK/dV) alone: 32 items of 64 steps took 1020 us in float32 dK/dV,
+// where 1152 steps on 256 CUs are 72 us of work. Such launches cut every item
+// into chunks of `per` steps, one workgroup each, with float32 partials that a
+// second kernel sums.
+//
+// plan_split returns the steps per chunk, or 0 to leave the items whole: the
+// chunk that minimises a model of the launch time,
+//   rounds of 256 workgroups x (start + per x step) + (kSplitLaunch + partial
+//   bytes written and read back),
+// against the whole items' start + step x (the longest item's steps, or a CU's
+// share of all steps where that is more). Step times are measured, one
+// workgroup per CU (two resident ones take about twice as long per step, so
+// counting 256 at a time prices them alike). grid(per): the workgroups of that
+// chunk; min_per: the chunk's granularity.
+// ---------------------------------------------------------------------------
+struct StepCost {
+  double fwd, dq, dkv;  // us per step (64 keys, 64 keys, 128 or 64 query rows)
+};
+StepCost step_cost(int32_t dtype, int32_t head_dim) {
+  if (dtype == PF_DTYPE_F32) return head_dim == 64 ? StepCost{4.6, 6.6, 8.0} : StepCost{9.0, 13.0, 16.0};
+  if (head_dim == 64) return {0.6, 0.9, 2.0};
+  if (head_dim == 256) return {2.0, 3.2, 3.9};
+  return {1.0, 1.5, 3.8};
+}
+constexpr double kStartUs = 5.0;        // a workgroup's prologue and epilogue
+constexpr double kSplitLaunchUs = 5.0;  // the second kernel
+constexpr double kPartialBytesPerUs = 4.0e6;
+constexpr int kCus = 256;
+constexpr int kMaxSplit = 64;
+
+template <typename F>
+int plan_split(int64_t items, int max_steps, double total_steps, int min_per, double step_us, int64_t partial_bytes,
+               F grid) {
+  if (items <= 0 || items >= 2 * kCus) return 0;
+  double best = kStartUs + step_us * fmax((double)max_steps, total_steps / kCus);
+  int best_per = 0, last = 0;
+  for (int n = 2; n <= kMaxSplit; n += 1 + n / 8) {
+    int per = (max_steps + n - 1) / n;
+    per = (per + min_per - 1) / min_per * min_per;
+    if (per >= max_steps || per == last) continue;
+    last = per;
+    const double wgs = (double)grid(per);
+    const double us = ceil(wgs / kCus) * (kStartUs + per * step_us) + kSplitLaunchUs +
+                      2.0 * wgs / (double)items * (double)partial_bytes / kPartialBytesPerUs;
+    if (us < 0.95 * best) {
+      best = us;
+      best_per = per;
+    }
+  }
+  return best_per;
+}
+
+size_t align_ws(size_t x) { return (x + 255) & ~(size_t)255; }
+
+// Key blocks of 64 summed over query blocks of `rows` rows (one head, one
+// batch): all of kv_len, or up to the block's diagonal.
+double sum_key_blocks(int Sq, int rows, int kv_len, bool causal) {
+  const int nq = (Sq + rows - 1) / rows;
+  if (!causal) return (double)nq * ((kv_len + 63) / 64);
+  double t = 0;
+  for (int i = 0; i < nq; ++i) {
+    const int64_t end = (int64_t)(i + 1) * rows;
+    const int e = (int)(end < Sq ? end : Sq);
+    t += ((e < kv_len ? e : kv_len) + 63) / 64;
+  }
+  return t;
+}
+
+int chunks_of(int q0, int rows, int Sq, int kv_len, int chunk, bool causal) {
+  return causal ? pf::key_chunks<true>(q0, rows, Sq, kv_len, chunk) : pf::key_chunks<false>(q0, rows, Sq, kv_len, chunk);
+}
+
+// The forward's key split: chunk and n_split of `p`, and its workspace bytes
+// (0: whole items).
+size_t plan_fwd_split(const pf_attn_fwd_args* a, pf::FwdParams* p) {
+  p->n_split = 1;
+  p->chunk = 0;
+  if (p->n_work == 0 || p->n_work >= 2 * kCus) return 0;
+  const int max_keys = a->causal && a->seq_len_q < a->kv_len ? a->seq_len_q : a->kv_len;
+  const int max_steps = (max_keys + 63) / 64;
+  if (max_steps <= 1) return 0;
+  const int64_t rows = (int64_t)a->batch * a->num_heads * a->seq_len_q;
+  const double total = sum_key_blocks(a->seq_len_q, p->rpw, a->kv_len, a->causal != 0) * (p->n_work / p->n_qblk);
+  const int min_per = a->causal && p->rpw > 64 ? 2 : 1;  // whole multiples of rpw
+  const auto grid = [&](int per) {
+    int64_t n = 0;
+    for (int i = 0; i < p->n_qblk; ++i) n += chunks_of(i * p->rpw, p->rpw, a->seq_len_q, a->kv_len, 64 * per, a->causal);
+    return n * (p->n_work / p->n_qblk);
+  };
+  const int per = plan_split(p->n_work, max_steps, total, min_per, step_cost(a->dtype, a->head_dim).fwd,
+                             rows * a->head_dim * 4, grid);
+  if (per == 0) return 0;
+  p->chunk = per * 64;
+  p->split_grid = (int)grid(per);
+  p->n_split = (max_steps + per - 1) / per;
+  const size_t prow = (size_t)p->n_split * rows;
+  return align_ws(prow * a->head_dim * 4) + align_ws(prow * 8);
+}
+
+void bind_fwd_split(const pf_attn_fwd_args* a, pf::FwdParams* p, void* ws) {
+  const size_t prow = (size_t)p->n_split * a->batch * a->num_heads * a->seq_len_q;
+  p->part_o = static_cast<float*>(ws);
+  p->part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + align_ws(prow * a->head_dim * 4));
 }
 
 // Minimum items for a dynamic tail: two per resident workgroup slot of a
@@ -197,6 +308,25 @@ int pf_attn_fwd(const pf_attn_fwd_args* a, void* stream) {
                                     (hipStream_t)stream));
 }
 
+size_t pf_attn_fwd_workspace_size(const pf_attn_fwd_args* a) {
+  pf::FwdParams p;
+  if (!a || fill_fwd(a, &p) != PF_OK) return 0;
+  return plan_fwd_split(a, &p);
+}
+
+int pf_attn_fwd_ws(const pf_attn_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!a) return PF_ERR_INVALID;
+  pf::FwdParams p;
+  int st = fill_fwd(a, &p);
+  if (st != PF_OK) return st;
+  if (p.n_work == 0) return PF_OK;
+  const size_t need = plan_fwd_split(a, &p);
+  if (need == 0) return pf_attn_fwd(a, stream);
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0) return PF_ERR_WORKSPACE;
+  bind_fwd_split(a, &p, workspace);
+  return finish(pf::launch_attn_fwd(p, a->dtype, a->head_dim, a->causal != 0, false, (hipStream_t)stream));
+}
+
 static size_t rope_ws_bytes(const pf_attn_fwd_args& b) {
   const size_t es = b.dtype == PF_DTYPE_F32 ? 4 : 2;
   return (((size_t)b.batch * b.num_kv_heads * b.seq_len_k * b.head_dim * es) + 255) & ~(size_t)255;
@@ -206,7 +336,7 @@ size_t pf_attn_fwd_rope_workspace_size(const pf_attn_fwd_rope_args* a) {
   if (!a) return 0;
   pf::FwdParams p;
   if (fill_fwd(&a->base, &p) != PF_OK) return 0;
-  return rope_ws_bytes(a->base);
+  return rope_ws_bytes(a->base) + plan_fwd_split(&a->base, &p);
 }
 
 int pf_attn_fwd_rope(const pf_attn_fwd_rope_args* a, void* stream) {
@@ -229,7 +359,11 @@ int pf_attn_fwd_rope(const pf_attn_fwd_rope_args* a, void* stream) {
   p.q_cos = a->q_cos;
   p.q_sin = a->q_sin;
   p.lse = nullptr;  // the reference's fused kernel has no LSE output
-  p.tail = plan_tail(p.n_work, kTwoPerCu, s);
+  // A workspace of the rotated K alone (a caller that sized it itself) runs
+  // whole items.
+  if (plan_fwd_split(&a->base, &p) > a->workspace_bytes - need) p.n_split = 1;
+  if (p.n_split > 1) bind_fwd_split(&a->base, &p, static_cast<char*>(a->workspace) + need);
+  else p.tail = plan_tail(p.n_work, kTwoPerCu, s);
   return finish(pf::launch_attn_fwd(p, a->base.dtype, a->base.head_dim, a->base.causal != 0, true, s));
 }
 
@@ -264,6 +398,9 @@ static int fill_bwd(const pf_attn_bwd_args* a, pf::BwdParams* p, bool need_grads
   p->sm_scale = a->sm_scale;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
   p->tail = pf::WorkTail{nullptr, 0, 0};
+  p->n_split_q = p->n_split_k = 1;
+  p->chunk_q = p->grid_q = p->steps_k = p->grid_k = 0;
+  p->part_dq = p->part_dk = p->part_dv = nullptr;
   const int64_t rows = (int64_t)a->batch * a->num_heads * a->seq_len_q;
   if (rows > kMaxGrid) return PF_ERR_UNSUPPORTED;
   // Per-(batch, head) byte offsets and buffer sizes are 32-bit inside the
@@ -297,6 +434,87 @@ int pf_attn_bwd_dkv(const pf_attn_bwd_args* a, void* stream) {
   if (st != PF_OK) return st;
   if ((int64_t)p.B * p.Hkv * p.Sk == 0) return PF_OK;
   return finish(pf::launch_attn_bwd_dkv(p, a->dtype, a->head_dim, a->causal != 0, (hipStream_t)stream));
+}
+
+// The backward's splits and their workspace: part_dq, part_dk, part_dv.
+static size_t plan_bwd_split(const pf_attn_bwd_args* a, pf::BwdParams* p, size_t* dq_bytes, size_t* dkv_bytes) {
+  *dq_bytes = *dkv_bytes = 0;
+  const StepCost cost = step_cost(a->dtype, a->head_dim);
+  const int64_t rows_q = (int64_t)p->B * p->Hq * p->Sq, rows_k = (int64_t)p->B * p->Hkv * p->Sk;
+  if (rows_q == 0 || rows_k == 0) return 0;
+  const bool causal = a->causal != 0;
+  const int max_keys = causal && p->Sq < p->kv_len ? p->Sq : p->kv_len;
+  const int kb = (max_keys + 63) / 64;
+  const int64_t dq_items = (int64_t)p->B * p->Hq * ((p->Sq + 127) / 128);
+  if (kb > 1 && dq_items < 2 * kCus) {
+    const double total = sum_key_blocks(p->Sq, 128, p->kv_len, causal) * p->B * p->Hq;
+    const auto grid = [&](int per) {
+      int64_t n = 0;
+      for (int q0 = 0; q0 < p->Sq; q0 += 128) n += chunks_of(q0, 128, p->Sq, p->kv_len, 64 * per, causal);
+      return n * p->B * p->Hq;
+    };
+    const int per = plan_split(dq_items, kb, total, 1, cost.dq, rows_q * a->head_dim * 4, grid);
+    if (per > 0) {
+      p->chunk_q = per * 64;
+      p->grid_q = (int)grid(per);
+      p->n_split_q = (kb + per - 1) / per;
+      *dq_bytes = align_ws((size_t)p->n_split_q * rows_q * a->head_dim * 4);
+    }
+  }
+  const int bmq = a->dtype != PF_DTYPE_F32 && a->head_dim <= 128 ? 128 : 64;
+  const int halves = a->head_dim > 128 ? 2 : 1;
+  const int64_t nk = (p->Sk + 127) / 128, items = (int64_t)p->B * p->Hkv * nk;
+  if (items * halves < 2 * kCus) {
+    const int64_t max_steps = (int64_t)((p->Sq + bmq - 1) / bmq) * p->g;
+    if (max_steps <= 0x7fffffff) {
+      double total = 0;
+      for (int64_t i = 0; i < nk; ++i) total += pf::dkv_steps(*p, (int)(128 * i), bmq, causal);
+      const auto grid = [&](int per) {
+        int64_t n = 0;
+        p->steps_k = per;
+        for (int64_t i = 0; i < nk; ++i) n += pf::dkv_runs(*p, (int)(128 * i), bmq, causal);
+        return n * p->B * p->Hkv * halves;
+      };
+      const int per = plan_split(items * halves, (int)max_steps, total * p->B * p->Hkv * halves, 1, cost.dkv,
+                                 2 * rows_k * a->head_dim * 4, grid);
+      p->steps_k = per;
+      if (per > 0) {
+        p->grid_k = (int)(grid(per) / halves);
+        p->n_split_k = (int)((max_steps + per - 1) / per);
+        *dkv_bytes = align_ws((size_t)p->n_split_k * rows_k * a->head_dim * 4);
+      }
+    }
+  }
+  return *dq_bytes + 2 * *dkv_bytes;
+}
+
+size_t pf_attn_bwd_workspace_size(const pf_attn_bwd_args* a) {
+  pf::BwdParams p;
+  if (fill_bwd(a, &p, true) != PF_OK) return 0;
+  size_t dq, dkv;
+  return plan_bwd_split(a, &p, &dq, &dkv);
+}
+
+int pf_attn_bwd_ws(const pf_attn_bwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  pf::BwdParams p;
+  int st = fill_bwd(a, &p, true);
+  if (st != PF_OK) return st;
+  size_t dq, dkv;
+  const size_t need = plan_bwd_split(a, &p, &dq, &dkv);
+  if (need == 0) return pf_attn_bwd(a, stream);
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255) != 0) return PF_ERR_WORKSPACE;
+  char* ws = static_cast<char*>(workspace);
+  p.part_dq = reinterpret_cast<float*>(ws);
+  p.part_dk = reinterpret_cast<float*>(ws + dq);
+  p.part_dv = reinterpret_cast<float*>(ws + dq + dkv);
+  hipStream_t s = (hipStream_t)stream;
+  if (p.n_split_q <= 1) p.tail = plan_tail(pf::bwd_dq_items(p), kTwoPerCu, s);
+  st = finish(pf::launch_attn_bwd_dq(p, a->dtype, a->head_dim, a->causal != 0, s));
+  if (st != PF_OK) return st;
+  p.tail = pf::WorkTail{nullptr, 0, 0};
+  st = finish(pf::launch_attn_bwd_dkv(p, a->dtype, a->head_dim, a->causal != 0, s));
+  if (st != PF_OK) return st;
+  return finish(pf::launch_attn_bwd_reduce(p, a->dtype, a->head_dim, a->causal != 0, s));
 }
 
 int pf_attn_bwd(const pf_attn_bwd_args* a, void* stream) {

@@ -79,6 +79,39 @@ __device__ inline int work_tail_item(const WorkTail& w, int n_work, int* lds) {
   return t < n_work - w.n_static ? w.n_static + t : -1;
 }
 
+// Workgroup `bid` of a split launch -> (block, member, chunk): the blocks (query
+// or key blocks) 0 .. n_blk - 1 have count(i) >= 1 chunks for each of `members`
+// items, and the grid holds exactly those workgroups, block after block (empty
+// ones would leave an XCD with more than its share: workgroups go round-robin
+// over the XCDs by index). The caller's blocks run heavy first. A lane takes a
+// block, so 64 blocks are one scan.
+struct SplitItem {
+  int blk, member, chunk;
+};
+template <typename F>
+__device__ inline SplitItem split_item(int bid, int n_blk, int members, F count) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int i0 = 0; i0 < n_blk; i0 += 64) {
+    const int n = i0 + lane < n_blk ? count(i0 + lane) : 0;
+    int incl = n * members;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    const int tot = __builtin_amdgcn_readlane(incl, 63);
+    if (bid < base + tot) {
+      const int ln = __builtin_ctzll(__ballot(base + incl > bid));
+      const int nb = __builtin_amdgcn_readlane(n, ln);
+      const int r = bid - base - (__builtin_amdgcn_readlane(incl, ln) - nb * members);
+      return SplitItem{i0 + ln, r / nb, r % nb};
+    }
+    base += tot;
+  }
+  return SplitItem{0, 0, 0};  // not reached: bid < the grid, the sum of the counts
+}
+
 // Forward prefill (optionally with fused RoPE).
 struct FwdParams {
   const void* q;
@@ -96,7 +129,30 @@ struct FwdParams {
   int n_work;        // B * Hq / hpw * n_qblk
   int pair_group;    // > 0: (batch, kv head) pairs an XCD streams at a time (fwd_work_item)
   WorkTail tail;
+  // Key split (n_split > 1, no tail): one workgroup per work item and chunk of
+  // `chunk` keys (a multiple of 64; causal: and of rpw) that its rows reach,
+  // n_split at most; split_grid workgroups in all.
+  int n_split;
+  int chunk;
+  int split_grid;
+  float* part_o;   // [n_split, B, Hq, Sq, D] float32, unnormalised
+  float* part_ml;  // [n_split, B, Hq, Sq, 2] (max in log2 units, sum)
 };
+
+// Chunks (of `chunk` keys) that query rows [q0, q0 + rows) reach, at least 1.
+template <bool CAUSAL>
+__host__ __device__ inline int key_chunks(int q0, int rows, int Sq, int kv_len, int chunk) {
+  int end = kv_len;
+  if (CAUSAL) {
+    const int e = q0 + rows < Sq ? q0 + rows : Sq;
+    end = e < end ? e : end;
+  }
+  return (end + chunk - 1) / chunk;
+}
+template <bool CAUSAL>
+__device__ inline int fwd_chunks(const FwdParams& p, int q0) {
+  return key_chunks<CAUSAL>(q0, p.rpw, p.Sq, p.kv_len, p.chunk);
+}
 
 // Work item of forward workgroup `bid`: (batch b, kv head kvh, head group hg
 // of the GQA group, query block qblk). Workgroups are dispatched round-robin
@@ -159,7 +215,34 @@ struct BwdParams {
   float sm_scale;
   float scale_log2;
   WorkTail tail;  // of the dQ kernel (the dK/dV kernel runs without one)
+  // Split work items (float32 partials, summed by the reduce kernel): dQ by
+  // chunks of chunk_q keys (n_split_q > 1, no tail), dK/dV by runs of steps_k
+  // steps of its loop (n_split_k > 1); grid_q, grid_k workgroups.
+  int n_split_q, chunk_q, grid_q;
+  int n_split_k, steps_k, grid_k;
+  float* part_dq;  // [n_split_q, B, Hq, Sq, D]
+  float* part_dk;  // [n_split_k, B, Hkv, Sk, D]
+  float* part_dv;
 };
+
+// Chunks of keys that the dQ work item of query rows [q0, q0 + 128) needs.
+template <bool CAUSAL>
+__device__ inline int dq_chunks(const BwdParams& p, int q0) {
+  return key_chunks<CAUSAL>(q0, 128, p.Sq, p.kv_len, p.chunk_q);
+}
+// Query rows per step of the dK/dV loop, and the steps of the work item of
+// keys [k0, k0 + 128): (group member, query block) pairs. Its runs of steps_k:
+// at least one (an item without steps writes zeros).
+template <typename T, int D>
+inline constexpr int kDkvRows = (sizeof(T) == 2 && D <= 128) ? 128 : 64;
+__host__ __device__ inline int dkv_steps(const BwdParams& p, int k0, int bmq, bool causal) {
+  const int q_begin = causal ? k0 / bmq * bmq : 0;
+  return (k0 < p.kv_len && q_begin < p.Sq) ? (p.Sq - q_begin + bmq - 1) / bmq * p.g : 0;
+}
+__host__ __device__ inline int dkv_runs(const BwdParams& p, int k0, int bmq, bool causal) {
+  const int n = (dkv_steps(p, k0, bmq, causal) + p.steps_k - 1) / p.steps_k;
+  return n > 1 ? n : 1;
+}
 
 // Work items of the dQ kernel (128 query rows of one head) and of the dK/dV
 // kernel (128 keys of one kv head, all its query heads).
@@ -171,6 +254,8 @@ hipError_t launch_attn_bwd_dq(const BwdParams& p, int dtype, int head_dim, bool 
                               hipStream_t stream);
 hipError_t launch_attn_bwd_dkv(const BwdParams& p, int dtype, int head_dim, bool causal,
                                hipStream_t stream);
+// Sum the partials of whichever of dQ and dK/dV was split (pf_attn_bwd_reduce_kernel).
+hipError_t launch_attn_bwd_reduce(const BwdParams& p, int dtype, int head_dim, bool causal, hipStream_t stream);
 
 // Split-KV single-query decode, contiguous cache or paged pool.
 struct DecodeParams {

@@ -121,12 +121,16 @@ class Tuning(ctypes.Structure):
 # (symbol, argtypes, restype) for every entry point the header declares.
 SIGNATURES = {
     "pf_attn_fwd": ([ctypes.POINTER(FwdArgs), c_ptr], ctypes.c_int),
+    "pf_attn_fwd_workspace_size": ([ctypes.POINTER(FwdArgs)], ctypes.c_size_t),
+    "pf_attn_fwd_ws": ([ctypes.POINTER(FwdArgs), c_ptr, ctypes.c_size_t, c_ptr], ctypes.c_int),
     "pf_attn_fwd_rope_workspace_size": ([ctypes.POINTER(FwdRopeArgs)], ctypes.c_size_t),
     "pf_attn_fwd_rope": ([ctypes.POINTER(FwdRopeArgs), c_ptr], ctypes.c_int),
     "pf_attn_bwd_delta": ([ctypes.POINTER(BwdArgs), c_ptr], ctypes.c_int),
     "pf_attn_bwd_dq": ([ctypes.POINTER(BwdArgs), c_ptr], ctypes.c_int),
     "pf_attn_bwd_dkv": ([ctypes.POINTER(BwdArgs), c_ptr], ctypes.c_int),
     "pf_attn_bwd": ([ctypes.POINTER(BwdArgs), c_ptr], ctypes.c_int),
+    "pf_attn_bwd_workspace_size": ([ctypes.POINTER(BwdArgs)], ctypes.c_size_t),
+    "pf_attn_bwd_ws": ([ctypes.POINTER(BwdArgs), c_ptr, ctypes.c_size_t, c_ptr], ctypes.c_int),
     "pf_attn_decode_workspace_size": ([ctypes.POINTER(DecodeArgs)], ctypes.c_size_t),
     "pf_attn_decode": ([ctypes.POINTER(DecodeArgs), c_ptr], ctypes.c_int),
     "pf_paged_attn_workspace_size": ([ctypes.POINTER(PagedArgs)], ctypes.c_size_t),

@@ -70,8 +70,11 @@ def _fwd(q, k, v, causal: bool, sm_scale: float, kv_len: int, want_lse: bool):
     args = _lib.FwdArgs(
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(lse),
         B, Hq, Hkv, Sq, Sk, D, kv_len, int(bool(causal)), float(sm_scale), _lib.dtype_tag(q))
+    L = _lib.lib()
+    ws_bytes = L.pf_attn_fwd_workspace_size(args)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with torch.cuda.device(q.device):
-        _lib.check(_lib.lib().pf_attn_fwd(args, _lib.stream_of(q)), "flash_attention forward")
+        _lib.check(L.pf_attn_fwd_ws(args, _lib.ptr(ws), ws_bytes, _lib.stream_of(q)), "flash_attention forward")
     return o, lse
 
 
@@ -89,8 +92,11 @@ def _bwd(q, k, v, o, lse, do, causal: bool, sm_scale: float, kv_len: int):
         _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(do), _lib.ptr(lse),
         _lib.ptr(delta), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
         B, Hq, Hkv, Sq, Sk, D, kv_len, int(bool(causal)), float(sm_scale), _lib.dtype_tag(q))
+    L = _lib.lib()
+    ws_bytes = L.pf_attn_bwd_workspace_size(args)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
     with torch.cuda.device(q.device):
-        _lib.check(_lib.lib().pf_attn_bwd(args, _lib.stream_of(q)), "flash_attention backward")
+        _lib.check(L.pf_attn_bwd_ws(args, _lib.ptr(ws), ws_bytes, _lib.stream_of(q)), "flash_attention backward")
     return dq, dk, dv
 
 
