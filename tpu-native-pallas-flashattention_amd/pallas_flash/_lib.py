@@ -169,6 +169,26 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The C++ host side of the public calls (csrc/torch_calls.cpp). Each of
+    its functions returns None for anything but the plain case, and the caller
+    then runs its general path."""
+    global _calls
+    if _calls is None:
+        lib()
+        try:
+            from . import _torch_calls
+        except ImportError as e:
+            raise RuntimeError(
+                "_torch_calls.so is not built (or not for this torch); run `make` in "
+                "tpu-native-pallas-flashattention_amd/ or __graft_entry__.build()") from e
+        _calls = _torch_calls
+    return _calls
+
+
 def check(status: int, what: str) -> None:
     """Map a pf_status to a Python exception."""
     if status == PF_OK:

@@ -147,6 +147,9 @@ def flash_attention_decode_step(
     Returns:
         ``[batch, num_heads, 1, head_dim]`` in q's dtype.
     """
+    o = _lib.calls().step(q, k_new, v_new, k_cache, v_cache, positions, cos, sin, ring, sm_scale)
+    if o is not None:
+        return o
     if q.dim() != 4 or q.shape[2] != 1:
         raise ValueError(f"decode step expects q of shape [batch, heads, 1, head_dim], got {tuple(q.shape)}")
     if k_cache.dim() != 4 or k_cache.shape != v_cache.shape:

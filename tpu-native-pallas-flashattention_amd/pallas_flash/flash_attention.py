@@ -150,6 +150,9 @@ def flash_attention(
         ``[batch, num_heads, seq_len_q, head_dim]`` in q's dtype. Differentiable
         in q, k, v (gradients in each input's dtype).
     """
+    o = _lib.calls().attention(q, k, v, causal, sm_scale, kv_len)
+    if o is not None:
+        return o
     kv_len = _validate(q, k, v, kv_len)
     head_dim = q.shape[3]
     if sm_scale is None:
@@ -220,6 +223,9 @@ def flash_attention_decode(
     Returns:
         ``[batch, num_heads, 1, head_dim]``.
     """
+    o = _lib.calls().decode(q, k_cache, v_cache, cache_len, sm_scale)
+    if o is not None:
+        return o
     if q.shape[2] != 1:
         raise ValueError(f"decode expects a single query row, got seq_len_q={q.shape[2]}")
     if any(t.requires_grad for t in (q, k_cache, v_cache)) and torch.is_grad_enabled():

@@ -126,6 +126,9 @@ def flash_attention_rope(
         causal, sm_scale, kv_len: as ``flash_attention``.
         block_q, block_k, interpret: accepted for compatibility; ignored.
     """
+    o = _lib.calls().rope(q, k, v, q_cos, q_sin, k_cos, k_sin, causal, sm_scale, kv_len)
+    if o is not None:
+        return o
     # fused_rope.py:154-181
     if k_cos is None or k_sin is None:
         if k.shape[2] != q.shape[2]:

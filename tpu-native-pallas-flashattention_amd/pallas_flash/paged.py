@@ -55,6 +55,9 @@ def paged_flash_attention(
         mixed dtypes copy the pool padded/cast per call, with a one-time
         warning (``_shape``).
     """
+    o = _lib.calls().paged(q, k_pages, v_pages, block_tables, context_lens, sm_scale)
+    if o is not None:
+        return o
     # paged.py:129-149
     if q.dim() != 4 or q.shape[2] != 1:
         raise ValueError(
