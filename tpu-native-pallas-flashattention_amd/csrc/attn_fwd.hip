@@ -59,7 +59,7 @@ constexpr int kFwdBN = 64;   // keys per block
 // of 512 rows and keys at head_dim 128: 32 whole items ran 73 us on 32 of 256
 // CUs.
 template <typename T, int D, bool CAUSAL, bool ROPE, bool SPLIT = false>
-__global__ __launch_bounds__(256, (kWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdParams p) {
+__global__ __launch_bounds__(256, (kFwdWgPerCu<T, D>)) void pf_attn_fwd_kernel(FwdParams p) {
   using MF = Mfma32<T>;
   using Frag = typename MF::Frag;
   using G = Tile<T, D>;

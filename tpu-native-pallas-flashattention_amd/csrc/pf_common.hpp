@@ -138,6 +138,13 @@ __device__ inline float keep_if_bit(float v, uint32_t m, int i) {
 // workgroup more than half the LDS, else 2.
 template <typename T, int D>
 inline constexpr int kWgPerCu = ((sizeof(T) == 4 && D == 128) || D > 128) ? 1 : 2;
+// The forward at 16-bit head_dim 64: three. Its exp and row-sum VALU work is
+// twice as long per MFMA as at head_dim 128, and the third wave of a SIMD hides
+// more of it than the two registers it gives up cost (B=8, 12 heads, S=1000:
+// 27.1 -> 25.4 us; B=4, 16 heads, S=2048: 47.9 -> 45 us). dQ would spill 11
+// registers there and ran 4-17% slower.
+template <typename T, int D>
+inline constexpr int kFwdWgPerCu = (sizeof(T) == 2 && D == 64) ? 3 : kWgPerCu<T, D>;
 
 // Reinterpret a 16-byte chunk as operand fragment i.
 template <typename T>

@@ -127,6 +127,7 @@ struct FwdParams {
   int rpw;           // query rows per head per workgroup (128 / hpw: 32 per wave)
   int n_qblk;        // ceil(Sq / rpw)
   int n_work;        // B * Hq / hpw * n_qblk
+  int snake;         // all items resident at once: odd rounds of 256 run light first
   int pair_group;    // > 0: (batch, kv head) pairs an XCD streams at a time (fwd_work_item)
   WorkTail tail;
   // Key split (n_split > 1, no tail): one workgroup per work item and chunk of
@@ -167,6 +168,8 @@ __device__ inline int fwd_chunks(const FwdParams& p, int q0) {
 // Both are bijections of [0, n_work).
 __device__ inline void fwd_work_item(int bid, const FwdParams& p, int& b, int& kvh, int& hg, int& qblk) {
   const int n_hg = p.g / p.hpw;
+  // every other whole round of 256 (32 workgroups of each XCD) back to front
+  if (p.snake && (bid >> 8 & 1) != 0 && (bid | 255) < p.n_work) bid ^= 0xf8;
   if (p.pair_group > 0) {
     const int per_pair = p.n_qblk * n_hg;
     const int P = p.pair_group;
