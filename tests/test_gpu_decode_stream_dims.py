@@ -5,7 +5,8 @@ The same partition logic as the 16-bit head_dim 128 kernel
 LDS bank window, 8 rows a load), 512-byte rows (16-key stages) and float32
 products, at the edges of their stages and page groups, on grids that leave
 sequences whole, cut in a few pieces and cut in one piece per stage (each
-combine form). Oracle: flash_attention.py:555-589 decode on the cache prefix,
+combine form), and at the ends of the form that gives a short sequence a
+workgroup of its own. Oracle: flash_attention.py:555-589 decode on the cache prefix,
 paged.py:45-99 over the gathered pages.
 """
 
@@ -31,12 +32,15 @@ def _waves(w):
 
 
 @pytest.mark.parametrize("w", [None, 1, 7])
-@pytest.mark.parametrize("dt,D", FORMS)
+@pytest.mark.parametrize("dt,D", FORMS + [("bf16", 128)])
 @pytest.mark.parametrize("B,Hq,Hkv,cap,L", [
     (3, 8, 2, 70, 1),       # one key; g = 4
     (2, 10, 2, 64, 15),     # g = 5: 16 query rows, a short 16-key stage
     (2, 32, 2, 64, 33),     # g = 16: every query row; one key past a stage
     (1, 1, 1, 1300, 1299),  # one sequence cut in dozens of pieces
+    (2, 8, 2, 400, 192),    # 12 stages of 16 keys: the last length of a workgroup per sequence there
+    (2, 8, 2, 400, 384),    # 12 stages of 32 keys
+    (2, 8, 2, 400, 385),    # one key more: the persistent grid
     (2, 34, 2, 40, 17),     # g = 17: the generic kernel
 ])
 def test_decode(w, dt, D, B, Hq, Hkv, cap, L):

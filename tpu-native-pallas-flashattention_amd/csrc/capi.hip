@@ -576,6 +576,7 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   p->stages = ns;
   const int wv = t.decode_waves.load(std::memory_order_relaxed);
   const int group = p->Hq / p->Hkv;
+  p->fixed_grid = wv > 0;
   p->n_waves = wv > 0 ? wv : pf::decode_stream_waves(dtype, p->D, ns, group);
   const int unit = dtype == PF_DTYPE_F32 && p->D == 128 ? 16 : 32;
   const int64_t runs = (int64_t)p->B * p->Hkv * ((group + 15) / 16) * ((max_len + unit - 1) / unit);

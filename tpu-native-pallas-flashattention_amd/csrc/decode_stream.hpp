@@ -387,8 +387,13 @@ __device__ inline int64_t wave_plan(const DecodeParams& p, int J, int W, int w, 
 // head slice 0 writes them to the cache slot. Every wave that reads the slot
 // (one per head slice) patches its own copy, so no wave depends on another's
 // global write within the launch.
-template <typename T, int D, int PG, int NS, int QR>
-__global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
+//
+// NWV = 1: the persistent grid of one-wave workgroups described above. NWV = 4
+// (short sequences, few of them): a workgroup per sequence, its four waves
+// taking a quarter of the stages each and merging through LDS at the end, so
+// no piece leaves the workgroup and no second kernel runs.
+template <typename T, int D, int PG, int NS, int QR, int NWV = 1>
+__global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams p) {
   using MF = Mfma16<T>;
   using G = StreamGeo<T, D>;
   constexpr int SK = G::SK, RB = G::RB, KPL = G::KPL, NU = G::NU, NL = G::NL, RPL = G::RPL;
@@ -396,9 +401,11 @@ __global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
   constexpr int kSlotB = G::slot_bytes(QR);
   static_assert(PG != 1 || (D == 128 && !G::F32), "the decode step is written for 16-bit 128-column rows");
   static_assert(PG <= 1 || (PG % RPL == 0 && SK % PG == 0), "a page group is whole loads of one stage");
-  __shared__ __attribute__((aligned(1024))) char smem[NS * kSlotB];
+  __shared__ __attribute__((aligned(1024))) char smem_all[NWV * NS * kSlotB];
 
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wv = NWV > 1 ? uni((int)(threadIdx.x >> 6)) : 0;
+  char* const smem = smem_all + wv * NS * kSlotB;  // this wave's ring
   const int i16 = lane & 15;
   const int h = lane >> 4;
   const int g = p.Hq / p.Hkv;
@@ -408,8 +415,19 @@ __global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
   const int w = blockIdx.x;
 
   Cursor cc;
-  const int64_t n = wave_plan<PG, SK>(p, J, W, w, &cc);  // stages of this wave
-  if (n <= 0) return;
+  int64_t n;  // stages of this wave
+  [[maybe_unused]] int per = 0;  // NWV > 1: stages per wave (the last ones may have fewer or none)
+  if constexpr (NWV > 1) {
+    const int b = w / J;
+    cc = Cursor{b, w - b * J, 0, 0, seq_len<PG>(p, b)};
+    cc.nst = (cc.L + SK - 1) / SK;
+    per = (cc.nst + NWV - 1) / NWV;
+    cc.st = wv * per;
+    n = min(per, cc.nst - cc.st);
+  } else {
+    n = wave_plan<PG, SK>(p, J, W, w, &cc);
+    if (n <= 0) return;
+  }
 
   const uint32_t lds0 = lds_u32(smem);
   const T* Kb = static_cast<const T*>(p.k);
@@ -733,8 +751,6 @@ __global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
       // ---- end of a piece ---------------------------------------------------
       float l_tot = l_run + __shfl_xor(l_run, 16);
       l_tot += __shfl_xor(l_tot, 32);
-      const int kvh = cc.j / n_hc, hc = cc.j - kvh * n_hc;
-      const int qh = hc * 16 + i16;
       // column d0 and value r of the lane's q-th group of 4 outputs (NACC groups)
       auto out4 = [&](int q, int& d0) -> f32x4 {
         if constexpr (G::F32) {
@@ -746,6 +762,22 @@ __global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
           return acc[q];
         }
       };
+      if constexpr (NWV > 1) {
+        // this wave's ring is consumed: its piece goes there, for the merge
+        float* po = reinterpret_cast<float*>(smem);
+        if (i16 < QR) {
+#pragma unroll
+          for (int q = 0; q < G::NACC; ++q) {
+            int d0;
+            const f32x4 a = out4(q, d0);
+            *reinterpret_cast<f32x4*>(po + i16 * D + d0) = a;
+          }
+          if (h == 0) *reinterpret_cast<f32x2*>(po + QR * D + 2 * i16) = (f32x2){m_run, l_tot};
+        }
+        break;
+      }
+      const int kvh = cc.j / n_hc, hc = cc.j - kvh * n_hc;
+      const int qh = hc * 16 + i16;
       if (piece_st0 == 0 && cc.st == cc.nst - 1) {
         // The whole sequence: finish it here.
         if (qh < g) {
@@ -777,6 +809,45 @@ __global__ __launch_bounds__(64) void pf_decode_stream_kernel(DecodeParams p) {
       first_piece = false;
     }
     cursor_next<PG, SK>(cc, p, J);
+  }
+  if constexpr (NWV > 1) {
+    // o = sum_i acc_i 2^(m_i - M) / sum_i l_i 2^(m_i - M) over the waves' pieces
+    // (none: o = 0), 4 columns of a head's row per thread.
+    __syncthreads();
+    const int kvh = cc.j / n_hc, hc = cc.j - kvh * n_hc;
+    const int nq = min(QR, g - hc * 16);
+    T* const out = static_cast<T*>(p.o) + ((int64_t)cc.b * p.Hq + (int64_t)kvh * g + hc * 16) * D;
+    for (int i = threadIdx.x; i < nq * (D / 4); i += 64 * NWV) {
+      const int row = i / (D / 4), d0 = 4 * (i % (D / 4));
+      f32x2 ml[NWV];
+      float M = kNegInf;
+#pragma unroll
+      for (int v = 0; v < NWV; ++v) {
+        ml[v] = (f32x2){kNegInf, 0.f};
+        if (v * per < cc.nst)
+          ml[v] = *reinterpret_cast<const f32x2*>(reinterpret_cast<float*>(smem_all + v * NS * kSlotB) + QR * D +
+                                                  2 * row);
+        M = fmaxf(M, ml[v][0]);
+      }
+      const float Mu = (M == kNegInf) ? 0.f : M;
+      f32x4 o = (f32x4)(0.f);
+      float l = 0.f;
+#pragma unroll
+      for (int v = 0; v < NWV; ++v) {
+        if (v * per < cc.nst) {
+          const float wt = exp2f(ml[v][0] - Mu);
+          l += ml[v][1] * wt;
+          o += *reinterpret_cast<const f32x4*>(reinterpret_cast<float*>(smem_all + v * NS * kSlotB) + row * D + d0) *
+               wt;
+        }
+      }
+      const float inv = (l == 0.f) ? 0.f : 1.f / l;
+      typedef T v4 __attribute__((ext_vector_type(4)));
+      v4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = Elem<T>::from_f32(o[e] * inv);
+      *reinterpret_cast<v4*>(out + row * D + d0) = y;
+    }
   }
 }
 
@@ -943,8 +1014,31 @@ hipError_t launch_combine(const DecodeParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Short sequences (at most 12 stages: three a wave) and at most as many as are
+// resident at once run a workgroup each (NWV = 4). One launch instead of two, and
+// no trip of the pieces through memory: calls over 80-250 keys 8.0-9.8 us ->
+// 5.1-6.6 us; from about 16 stages the longer chain costs what the second
+// kernel did. A grid size set by hand (decode_waves) keeps the persistent grid.
+constexpr int kShortWaves = 4, kShortStages = 12;
+template <typename T, int D, int PG, int QR>
+bool short_form(const DecodeParams& p) {
+  using G = StreamGeo<T, D>;
+  const int64_t seqs = (int64_t)p.B * p.Hkv * ((p.Hq / p.Hkv + 15) / 16);
+  const int64_t len = PG <= 1 ? p.cache_len : (int64_t)p.pages_per_seq * p.page_size;
+  constexpr int per_cu = 160 * 1024 / (kShortWaves * 2 * G::slot_bytes(QR));
+  return per_cu > 0 && !p.fixed_grid && p.stages == 2 && seqs <= 256 * per_cu && len <= kShortStages * G::SK;
+}
+
 template <typename T, int D, int PG, int NS, int QR>
 hipError_t launch_stream(const DecodeParams& p, hipStream_t st) {
+  if constexpr (NS == 2 && kShortWaves * 2 * StreamGeo<T, D>::slot_bytes(QR) <= 160 * 1024) {
+    if (short_form<T, D, PG, QR>(p)) {
+      const unsigned seqs = (unsigned)(p.B * p.Hkv * ((p.Hq / p.Hkv + 15) / 16));
+      hipLaunchKernelGGL((pf_decode_stream_kernel<T, D, PG, 2, QR, kShortWaves>), dim3(seqs), dim3(64 * kShortWaves),
+                         0, st, p);
+      return hipGetLastError();
+    }
+  }
   hipLaunchKernelGGL((pf_decode_stream_kernel<T, D, PG, NS, QR>), dim3((unsigned)p.n_waves), dim3(64), 0, st, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

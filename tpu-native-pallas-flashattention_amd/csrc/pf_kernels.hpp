@@ -283,6 +283,7 @@ struct DecodeParams {
   int chunk;          // keys per chunk (multiple of 32)
   float scale_log2;
   int stages;         // streaming kernel: LDS ring depth (2..4)
+  int fixed_grid;     // n_waves was set by hand (tuning): keep the persistent grid
   int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
   // Fused decode step (streaming kernel, positions != null): the new token of
   // batch b is at pos = positions[b * pos_stride]; its k (rotated with table
