@@ -299,7 +299,7 @@ def bench_d256(L, _lib, torch, steps, warmup, iters):
     prefill = {"fwd_ms": ev.mean_ms(0, 1), "dq_ms": ev.mean_ms(1, 2), "dkv_ms": ev.mean_ms(2, 3),
                "step_ms": ev.mean_ms(0, 3), "F": F}
     del q, k, v, do, o, lse, delta, dq, dk, dv
-    # decode: config 4's shape at head_dim 256 (generic split-KV kernel)
+    # decode: config 4's shape at head_dim 256 (streaming kernel, 16-key stages)
     B, Hq, Hkv, cap, kv_len = 64, 32, 8, 8192, 6000
     qd = torch.randn((B, Hq, 1, D), generator=g, device="cuda").to(torch.bfloat16)
     kc = torch.empty((B, Hkv, cap, D), dtype=torch.bfloat16, device="cuda")

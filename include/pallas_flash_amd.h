@@ -218,10 +218,11 @@ int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspa
  *   k_cache, v_cache [batch, num_kv_heads, cache_size, head_dim]
  *   cache_len in (0, cache_size]; slots >= cache_len are never read.
  *   head_dim <= 256 (bf16/f16) or 128 (float32), a multiple of 8 (bf16/f16)
- *   or 4 (float32): rows are read in place; bf16/f16 with head_dim 128 run
- *   the streaming kernel, other head dims and float32 the generic kernel
- *   (computing at 64, 128 or 256 with the missing columns as zeros), with
- *   the same results to rounding.
+ *   or 4 (float32): rows are read in place; head_dim 64, 128 and (bf16/f16)
+ *   256 run the streaming kernel -- off bf16/f16 head_dim 128, for groups of
+ *   at most 16 query heads per KV head --, other head dims and larger groups
+ *   the generic kernel (computing at 64, 128 or 256 with the missing columns
+ *   as zeros), with the same results to rounding.
  * workspace: at least pf_attn_decode_workspace_size(args) bytes, 256-byte
  * aligned device memory (contents on entry do not matter).
  * ------------------------------------------------------------------------- */
@@ -252,10 +253,10 @@ int pf_attn_decode(const pf_attn_decode_args* args, void* stream);
  * non-positive length gives o = 0. Table entries at logical pages at or past
  * ceil(len / page_size) are never read (so -1 padding is legal); live entries
  * are clamped into [0, num_pages). Any page_size >= 1 is accepted (the
- * reference has no restriction). head_dim as pf_attn_decode. bf16/f16 with
- * head_dim 128 and page_size a multiple of 4 run the streaming kernel (each
- * 4-row load stays inside one page); other page sizes, dtypes and head dims
- * run the generic split-KV kernel, with the same results to rounding.
+ * reference has no restriction). head_dim and kernels as pf_attn_decode; the
+ * streaming kernel takes page sizes that are a multiple of 4 (of 8 for bf16/f16
+ * at head_dim 64), so that a load stays inside one page, the generic split-KV
+ * kernel the others, with the same results to rounding.
  * workspace: at least pf_paged_attn_workspace_size(args) bytes.
  * ------------------------------------------------------------------------- */
 typedef struct {
@@ -287,9 +288,10 @@ int pf_paged_attn(const pf_paged_attn_args* args, void* stream);
  * process ends.
  *  - A call whose partials need more than PF_NOALLOC_SCRATCH_BYTES
  *    (pf_paged_attn_workspace_size(args) larger) returns PF_ERR_WORKSPACE
- *    and enqueues nothing. bf16/f16, head_dim 128, page_size % 4 == 0 (the
- *    streaming kernel) needs at most about 16.3 MiB at the default tuning on
- *    a 256-CU device, whatever the batch; the generic kernel needs about
+ *    and enqueues nothing. The streaming kernel (pf_paged_attn) needs at most
+ *    about 16.5 MiB (bf16/f16 head_dim 256 with more than 4 heads per KV head:
+ *    24.2 MiB) at the default tuning on a 256-CU device, whatever the batch; the
+ *    generic kernel needs about
  *    batch * num_heads * splits * 520 bytes.
  *  - A call uses the array of the device `stream` belongs to (the null
  *    stream's: the current device).
