@@ -583,6 +583,13 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   if (p->n_waves > runs) p->n_waves = (int)(runs > 1 ? runs : 1);
   p->n_split = 0;
   p->chunk = 0;
+  p->g = group;
+  if (p->block_tables == nullptr && p->positions == nullptr && p->context_lens == nullptr) {
+    const int row_bytes = p->D * (dtype == PF_DTYPE_F32 ? 4 : 2), sk = row_bytes == 512 ? 16 : 32;
+    const int64_t stages = (int64_t)p->B * p->Hkv * ((group + 15) / 16) * ((max_len + sk - 1) / sk);
+    p->part_q = stages / p->n_waves;
+    p->part_rem = stages % p->n_waves;
+  }
   return p->n_waves;
 }
 

@@ -226,6 +226,7 @@ __device__ inline int64_t div_pos(int64_t a, int b, int64_t* rem) {
 struct Partition {
   int64_t q, rem;
   __device__ inline Partition(int64_t S, int W) { q = div_pos(S, W, &rem); }
+  __device__ inline Partition(int64_t q_, int64_t rem_) : q(q_), rem(rem_) {}
   __device__ inline int64_t start(int w) const { return (int64_t)w * q + min((int64_t)w, rem); }
   __device__ inline int wave_of(int64_t s) const {
     int64_t r;
@@ -275,7 +276,10 @@ __device__ inline int64_t locate(const DecodeParams& p, int J, int64_t s, Cursor
     if (s >= 0) {
       int64_t r, st;
       int b;
-      if ((per_b >> 31) == 0) {
+      if (p.B == 1) {
+        b = 0;
+        r = s;
+      } else if ((per_b >> 31) == 0) {
         b = (int)div_pos(s, (int)per_b, &r);
       } else {
         b = (int)(s / per_b);
@@ -341,6 +345,18 @@ __device__ inline Lens64 lens64(const DecodeParams& p, int J) {
   return r;
 }
 
+// The partition of all batches' stages: one length for all (PG == 0), the host
+// divided; otherwise a scan of the lengths.
+template <int PG, int SK>
+__device__ inline Partition partition(const DecodeParams& p, int J, int W) {
+  if constexpr (PG == 0) {
+    return Partition(p.part_q, p.part_rem);
+  } else {
+    Cursor unused;
+    return Partition(locate<PG, SK>(p, J, -1, &unused), W);
+  }
+}
+
 // The stages of wave w of W: their count (returned) and, if any, the cursor
 // of the first one.
 template <int PG, int SK>
@@ -362,7 +378,7 @@ __device__ inline int64_t wave_plan(const DecodeParams& p, int J, int W, int w, 
     }
     return n;
   }
-  const Partition part(locate<PG, SK>(p, J, -1, cc), W);
+  const Partition part = partition<PG, SK>(p, J, W);
   const int64_t s0 = part.start(w);
   const int64_t n = part.start(w + 1) - s0;
   if (n > 0) locate<PG, SK>(p, J, s0, cc);
@@ -408,7 +424,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
   char* const smem = smem_all + wv * NS * kSlotB;  // this wave's ring
   const int i16 = lane & 15;
   const int h = lane >> 4;
-  const int g = p.Hq / p.Hkv;
+  const int g = p.g;
   const int n_hc = (g + 15) >> 4;
   const int J = p.Hkv * n_hc;
   const int W = p.n_waves;
@@ -449,7 +465,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
   auto issue = [&](const Cursor& c, int slot, bool with_q) {
     const uint32_t ldk = lds0 + (uint32_t)(slot * kSlotB);
     const uint32_t ldv = ldk + G::TILE;
-    const int kvh = c.j / n_hc, hc = c.j - kvh * n_hc;
+    const int kvh = n_hc == 1 ? c.j : c.j / n_hc, hc = c.j - kvh * n_hc;
     if (with_q) {
       const int q0 = hc * 16;
       const int nq = min(QR, g - q0);
@@ -512,7 +528,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
   };
   [[maybe_unused]] auto step_load = [&](const Cursor& c, StepData& d) {
     d.pos = sload_i32(p.positions, (int64_t)c.b * p.pos_stride);  // valid: the piece has keys
-    const int kvh = c.j / n_hc;
+    const int kvh = n_hc == 1 ? c.j : c.j / n_hc;
     const int64_t src = ((int64_t)c.b * p.Hkv + kvh) * 128;
     if (lane < 32) {
       const T* nb = static_cast<const T*>(lane < 16 ? p.k_new : p.v_new) + src;
@@ -571,7 +587,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
     if (lane < 32) {
       char* t = lane < 16 ? tK : tV;
       sts16(t + r * RB + 16 * (i16 ^ G::swz(r)), row);
-      const int kvh = c.j / n_hc, hc = c.j - kvh * n_hc;
+      const int kvh = n_hc == 1 ? c.j : c.j / n_hc, hc = c.j - kvh * n_hc;
       if (hc == 0) {
         T* out = static_cast<T*>(lane < 16 ? p.k_out : p.v_out);
         stg16(out + (((int64_t)c.b * p.Hkv + kvh) * p.cache_size + tslot) * 128 + 8 * i16, row);
@@ -776,7 +792,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
         }
         break;
       }
-      const int kvh = cc.j / n_hc, hc = cc.j - kvh * n_hc;
+      const int kvh = n_hc == 1 ? cc.j : cc.j / n_hc, hc = cc.j - kvh * n_hc;
       const int qh = hc * 16 + i16;
       if (piece_st0 == 0 && cc.st == cc.nst - 1) {
         // The whole sequence: finish it here.
@@ -814,7 +830,7 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
     // o = sum_i acc_i 2^(m_i - M) / sum_i l_i 2^(m_i - M) over the waves' pieces
     // (none: o = 0), 4 columns of a head's row per thread.
     __syncthreads();
-    const int kvh = cc.j / n_hc, hc = cc.j - kvh * n_hc;
+    const int kvh = n_hc == 1 ? cc.j : cc.j / n_hc, hc = cc.j - kvh * n_hc;
     const int nq = min(QR, g - hc * 16);
     T* const out = static_cast<T*>(p.o) + ((int64_t)cc.b * p.Hq + (int64_t)kvh * g + hc * 16) * D;
     for (int i = threadIdx.x; i < nq * (D / 4); i += 64 * NWV) {
@@ -874,29 +890,28 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
   const int wv = uni((int)(threadIdx.x >> 6));
   const int bh = WPB == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
   if (WPB == 1 && bh >= p.B * p.Hq) return;
-  const int b = bh / p.Hq, hq = bh - b * p.Hq;
-  const int g = p.Hq / p.Hkv;
+  const int b = p.B == 1 ? 0 : bh / p.Hq, hq = bh - b * p.Hq;
+  const int g = p.g;
   const int n_hc = (g + 15) >> 4;
   const int J = p.Hkv * n_hc;
   const int kvh = hq / g, qh = hq - kvh * g, hc = qh >> 4, qi = qh & 15;
   const int W = p.n_waves;
 
   // Global stage range [s0, s1) of this head's sequence.
-  int64_t S, before = 0;  // all stages; stages of batches < b
+  Partition part((int64_t)0, (int64_t)0);  // of all stages
+  int64_t before = 0;     // stages of batches < b
   int L;
   if constexpr (PG == 0) {
-    Cursor dummy;
-    S = locate<PG, SK>(p, J, -1, &dummy);
+    part = partition<PG, SK>(p, J, W);
     L = p.cache_len;
     before = (int64_t)b * ((L + SK - 1) / SK) * J;
   } else if (p.B <= 64) {
     const Lens64 ls = lens64<PG, SK>(p, J);
-    S = ls.tot;
+    part = Partition(ls.tot, W);
     before = uni64(__shfl(ls.incl - ls.t, b));
     L = __builtin_amdgcn_readfirstlane(__shfl(ls.L, b));
   } else {
-    Cursor dummy;
-    S = locate<PG, SK>(p, J, -1, &dummy);
+    part = partition<PG, SK>(p, J, W);
     for (int b0 = 0; b0 < b; b0 += 64) {
       const int bb = b0 + lane;
       const int Lb = bb < b ? len_lane<PG>(p, bb) : 0;
@@ -917,7 +932,6 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
     }
     return;
   }
-  const Partition part(S, W);
   const int64_t s0 = before + (int64_t)(kvh * n_hc + hc) * nst;
   const int wa = uni(part.wave_of(s0)), wb = uni(part.wave_of(s0 + nst - 1));
   if (wa == wb) return;  // finished by the main kernel (uniform over the workgroup)

@@ -283,6 +283,8 @@ struct DecodeParams {
   int chunk;          // keys per chunk (multiple of 32)
   float scale_log2;
   int stages;         // streaming kernel: LDS ring depth (2..4)
+  int g;              // query heads per kv head (streaming kernel)
+  int64_t part_q, part_rem;  // contiguous cache: the stages of the call divided by n_waves
   int fixed_grid;     // n_waves was set by hand (tuning): keep the persistent grid
   int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
   // Fused decode step (streaming kernel, positions != null): the new token of
