@@ -84,3 +84,23 @@ def test_paged(w, dt, D, page):
     clean = lambda t: np.nan_to_num(host(t))
     check_fwd(out, paged_ref(host(tq), clean(tk), clean(tv), np.where(table < 0, 0, table), lens), dt)
     assert (out[0] == 0).all()
+
+
+@pytest.mark.parametrize("dt,D", [("f16", 64), ("bf16", 256), ("f32", 128)])
+def test_unaligned_cache_keeps_the_generic_kernel(dt, D):
+    """A contiguous cache that starts between two 16-byte boundaries: the
+    streaming kernel's loads want aligned rows, so the generic kernel reads it."""
+    note(f"unaligned cache {dt} D={D}")
+    rng = np.random.default_rng(D)
+    B, Hq, Hkv, cap, L = 2, 8, 2, 300, 290
+    tq = dev(rng.standard_normal((B, Hq, 1, D)), dt)
+    caches = []
+    for _ in range(2):
+        x = dev(rng.standard_normal((B, Hkv, cap, D)), dt)
+        flat = torch.empty(x.numel() + 8, dtype=x.dtype, device="cuda")
+        view = flat[1:1 + x.numel()].view(x.shape)
+        view.copy_(x)
+        assert view.is_contiguous() and view.data_ptr() % 16 != 0
+        caches.append(view)
+    out = host(flash_attention_decode(tq, *caches, L))
+    check_fwd(out, decode_ref(host(tq), host(caches[0]), host(caches[1]), L), dt)

@@ -91,3 +91,21 @@ def test_chunk_of_minus_infinity_scores():
     out = flash_attention(q, k, v)
     want = flash_attention(q, k, v, kv_len=512)
     check_fwd(host(out), host(want), "f32")
+
+
+@pytest.mark.parametrize("B,H,S", [(8, 12, 1000), (5, 13, 1100), (3, 11, 1025)])
+def test_resident_causal_items(B, H, S):
+    """16-bit head_dim 64, causal, 257-768 work items (no split, every other
+    round of 256 back to front; whole and partial last rounds): every row against
+    the float32 product."""
+    n_work = B * H * -(-S // 128)
+    assert 256 < n_work <= 768
+    note(f"resident causal items B={B} H={H} S={S}")
+    g = torch.Generator("cuda").manual_seed(S)
+    q, k, v = (torch.randn((B, H, S, 64), device="cuda", generator=g).half() for _ in range(3))
+    out = flash_attention(q, k, v, causal=True)
+    mask = torch.ones((S, S), dtype=torch.bool, device="cuda").triu_(1)
+    for b in range(B):
+        s = torch.matmul(q[b].float(), k[b].float().transpose(1, 2).contiguous()) * 0.125
+        ref = torch.matmul(torch.softmax(s.masked_fill_(mask, -float("inf")), -1), v[b].float())
+        check_fwd(host(out[b]), host(ref), "f16")

@@ -598,8 +598,12 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
 static bool stream_range_ok(int64_t rows, int32_t head_dim, int32_t dtype) {
   return rows * head_dim * (dtype == PF_DTYPE_F32 ? 4 : 2) < ((int64_t)1 << 31);
 }
+// Its LDS loads want 16-byte aligned rows; the generic kernel reads any.
+static bool stream_aligned(const void* q, const void* k, const void* v) {
+  return (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+}
 // The 16-bit head_dim 128 forms run on the streaming kernel alone; the others
-// fall back to the generic kernel past its range.
+// fall back to the generic kernel past its range and for unaligned operands.
 static bool stream_only(int32_t head_dim, int32_t dtype) { return head_dim == 128 && dtype != PF_DTYPE_F32; }
 
 static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
@@ -628,7 +632,8 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, false, 0)) {
     // buffer offsets within one (b, kv head) run are 32-bit
-    if (stream_range_ok(a->cache_size, a->head_dim, a->dtype)) {
+    if (stream_range_ok(a->cache_size, a->head_dim, a->dtype) &&
+        (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_cache, a->v_cache))) {
       if (stream_setup(p, a->dtype, a->cache_len) <= 0) return PF_ERR_LAUNCH;
       return PF_OK;
     }
@@ -714,7 +719,8 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p) {
   p->pages_per_seq = a->pages_per_seq;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, true, a->page_size)) {
-    if (stream_range_ok(a->page_size, a->head_dim, a->dtype)) {
+    if (stream_range_ok(a->page_size, a->head_dim, a->dtype) &&
+        (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_pages, a->v_pages))) {
       if (stream_setup(p, a->dtype, max_len) <= 0) return PF_ERR_LAUNCH;
       return PF_OK;
     }
