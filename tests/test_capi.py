@@ -154,6 +154,16 @@ def test_decode_workspace_and_rejections(L):
     assert L.pf_attn_decode_workspace_size(_dec(num_heads=30)) == 0
 
 
+@pytest.mark.parametrize("heads,kv", [(16, 4), (16, 2)])
+def test_decode_workspace_of_a_longer_cache_serves_a_shorter_one(L, heads, kv):
+    """Also where a float32 call changes to shorter stages and more waves."""
+    ws = [L.pf_attn_decode_workspace_size(
+        _dec(q=256, k_cache=256, v_cache=256, dtype=0, head_dim=64, batch=20, num_heads=heads,
+             num_kv_heads=kv, cache_size=40000, cache_len=n))
+        for n in (1, 16, 384, 385, 400, 416, 417, 800, 833, 13088, 13120, 26208, 26240, 40000)]
+    assert ws == sorted(ws) and ws[0] > 0
+
+
 def _paged(**over):
     base = dict(q=8, k_pages=8, v_pages=8, block_tables=8, context_lens=8, o=8, batch=128,
                 num_heads=32, num_kv_heads=8, num_pages=16384, page_size=64, head_dim=128,

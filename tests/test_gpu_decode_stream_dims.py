@@ -86,6 +86,48 @@ def test_paged(w, dt, D, page):
     assert (out[0] == 0).all()
 
 
+@pytest.mark.parametrize("w", [None, 7])
+@pytest.mark.parametrize("B,Hq,Hkv,L", [
+    (20, 16, 4, 409),  # 80 x 13 stages of 32 keys: more than there are waves, 16-key stages
+    (20, 16, 4, 416),  # whole stages
+    (27, 10, 2, 593),  # g = 5: 16 query rows; one key past a 16-key stage
+    (20, 12, 3, 545),  # 60 x 18, one key into the last
+    (16, 8, 4, 512),   # 64 x 16: a 32-key stage each still
+])
+def test_f32_fine_stages(w, B, Hq, Hkv, L):
+    note(f"fine stages waves={w} B={B} Hq={Hq} Hkv={Hkv} L={L}")
+    rng = np.random.default_rng(L)
+    q = rng.standard_normal((B, Hq, 1, 64))
+    k, v = rng.standard_normal((2, B, Hkv, L + 3, 64))
+    k[:, :, L:] = v[:, :, L:] = np.nan
+    tq, tk, tv = dev(q, "f32"), dev(k, "f32"), dev(v, "f32")
+    with _waves(w):
+        out = host(flash_attention_decode(tq, tk, tv, L))
+    check_fwd(out, decode_ref(host(tq), host(tk), host(tv), L), "f32")
+
+
+@pytest.mark.parametrize("Hq", [4, 12])
+@pytest.mark.parametrize("page", [4, 8, 12, 16, 48, 64])
+def test_f32_fine_stages_paged(Hq, page):
+    """60 sequences x up to 576 keys, g = 2 and 6."""
+    note(f"fine stages paged Hq={Hq} page={page}")
+    rng = np.random.default_rng(page)
+    B, Hkv, pps = 30, 2, 576 // page
+    lens = rng.integers(0, 577, B).astype(np.int32)
+    lens[:6] = [0, 1, 15, 17, 33, 576]
+    table = rng.permutation(B * pps).reshape(B, pps).astype(np.int32)
+    q = rng.standard_normal((B, Hq, 1, 64))
+    kp, vp = rng.standard_normal((2, B * pps, Hkv, page, 64))
+    for b, n in enumerate(lens):
+        for j in range(pps):
+            kp[table[b, j], :, max(n - j * page, 0):] = vp[table[b, j], :, max(n - j * page, 0):] = np.nan
+    tq, tk, tv = dev(q, "f32"), dev(kp, "f32"), dev(vp, "f32")
+    out = host(paged_flash_attention(tq, tk, tv, torch.as_tensor(table), torch.as_tensor(lens)))
+    clean = lambda t: np.nan_to_num(host(t))
+    check_fwd(out, paged_ref(host(tq), clean(tk), clean(tv), table, lens), "f32")
+    assert (out[0] == 0).all()
+
+
 @pytest.mark.parametrize("dt,D", [("f16", 64), ("bf16", 256), ("f32", 128)])
 def test_unaligned_cache_keeps_the_generic_kernel(dt, D):
     """A contiguous cache that starts between two 16-byte boundaries: the

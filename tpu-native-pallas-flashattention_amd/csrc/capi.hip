@@ -5,6 +5,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -566,7 +567,7 @@ static int decode_chunk(int64_t units, int max_len) {
 // of the 16-bit head_dim 128 kernels) and decode_waves (grid size; any value
 // >= 1 is correct, only the resident count is fast).
 // A short problem starts only as many waves as it has stages (32 keys; 16 in
-// float32 at head_dim 128), and keeps no partial slots for more; at 16-bit
+// float32 at head_dim 128 and with fine stages), and keeps no partial slots for more; at 16-bit
 // head_dim 256 a wave takes at least two 16-key stages, which halves the slots
 // for 0.6 us. One stage a wave also cuts equal sequences alike, whatever
 // their place in the list. max_len: the most keys a sequence can have.
@@ -577,16 +578,33 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   const int wv = t.decode_waves.load(std::memory_order_relaxed);
   const int group = p->Hq / p->Hkv;
   p->fixed_grid = wv > 0;
-  p->n_waves = wv > 0 ? wv : pf::decode_stream_waves(dtype, p->D, ns, group);
-  const int unit = dtype == PF_DTYPE_F32 && p->D == 128 ? 16 : 32;
-  const int64_t runs = (int64_t)p->B * p->Hkv * ((group + 15) / 16) * ((max_len + unit - 1) / unit);
-  if (p->n_waves > runs) p->n_waves = (int)(runs > 1 ? runs : 1);
+  // Float32 at head_dim 64: a stage is 0.9 us of float32 MFMAs, so with a few
+  // stages a wave half as long ones, on twice as many waves (8 a CU), divide
+  // more evenly and hide each other's loads: 16 x 4 sequences of 64-2048 keys
+  // 16.0 -> 14.8 us, 8 x 8 of 1672 17.1 -> 14.7; past 32 stages a wave (by the
+  // longest lengths) nothing is left to gain and 190 a wave lose 2%. Where each
+  // 32-key stage has a wave of its own they only double the pieces to merge
+  // (8 sequences of 2447 keys 10.4 -> 11.5 us). Sequences of up to 12 stages
+  // have a form of their own.
+  const int64_t seqs = (int64_t)p->B * p->Hkv * ((group + 15) / 16);
+  const int64_t stages32 = seqs * ((max_len + 31) / 32);
+  const bool f32 = dtype == PF_DTYPE_F32, can_fine = f32 && p->D == 64;
+  p->fine = can_fine && max_len > 12 * 32 && stages32 > 4 * kCus && stages32 <= 32 * 4 * kCus;
+  const int sk = p->D * (f32 ? 4 : 2) == 512 || p->fine ? 16 : 32;  // keys per stage
+  auto waves = [&](bool fine, int unit) {
+    const int64_t runs = seqs * ((max_len + unit - 1) / unit);
+    const int n = wv > 0 ? wv : pf::decode_stream_waves(dtype, p->D, ns, group, fine);
+    return n > runs ? (int)(runs > 1 ? runs : 1) : n;
+  };
+  p->n_waves = waves(p->fine != 0, f32 ? sk : 32);
+  // Partials are sized for either choice, so that a workspace made for a long
+  // cache also serves a shorter one.
+  p->slot_waves = can_fine ? std::max(p->n_waves, waves(true, 16)) : p->n_waves;
   p->n_split = 0;
   p->chunk = 0;
   p->g = group;
   if (p->block_tables == nullptr && p->positions == nullptr && p->context_lens == nullptr) {
-    const int row_bytes = p->D * (dtype == PF_DTYPE_F32 ? 4 : 2), sk = row_bytes == 512 ? 16 : 32;
-    const int64_t stages = (int64_t)p->B * p->Hkv * ((group + 15) / 16) * ((max_len + sk - 1) / sk);
+    const int64_t stages = seqs * ((max_len + sk - 1) / sk);
     p->part_q = stages / p->n_waves;
     p->part_rem = stages % p->n_waves;
   }
@@ -651,7 +669,7 @@ static size_t decode_slots(const pf::DecodeParams& p) {
   if (p.n_waves > 0) {
     const int group = p.Hq / p.Hkv;
     const int64_t seqs = (int64_t)p.B * p.Hkv * ((group + 15) / 16);
-    return (size_t)(p.n_waves + (seqs < p.n_waves ? seqs : p.n_waves)) * pf::decode_stream_qrows(group);
+    return (size_t)(p.slot_waves + (seqs < p.slot_waves ? seqs : p.slot_waves)) * pf::decode_stream_qrows(group);
   }
   return (size_t)p.B * p.Hq * p.n_split;
 }

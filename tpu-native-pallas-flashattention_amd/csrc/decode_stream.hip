@@ -20,7 +20,7 @@ bool decode_stream_supported(int dtype, int head_dim, int group, bool paged, int
 }
 
 int stream_blocks_dims(int head_dim, bool small);
-int stream_blocks_f32(int head_dim, bool small);
+int stream_blocks_f32(int head_dim, bool small, bool fine);
 hipError_t launch_stream_dims(const DecodeParams& p, int dtype, bool paged, hipStream_t stream);
 hipError_t launch_stream_f32(const DecodeParams& p, bool paged, hipStream_t stream);
 
@@ -33,8 +33,9 @@ hipError_t launch_stream_f32(const DecodeParams& p, bool paged, hipStream_t stre
 namespace {
 
 constexpr int kMaxDevices = 64;
-// variants: 16-bit head_dim 128 at 2, 3, 4 stages; 16-bit 64, 256; float32 64, 128
-constexpr int kVariants = 7;
+// variants: 16-bit head_dim 128 at 2, 3, 4 stages; 16-bit 64, 256; float32 64,
+// 128; float32 64 with 16-key stages
+constexpr int kVariants = 8;
 
 struct StreamOccupancy {
   std::once_flag once;
@@ -56,19 +57,20 @@ void query_occupancy(StreamOccupancy* o, int dev) {
   for (int s = 0; s < 2; ++s) {
     o->per_cu[3][s] = stream_blocks_dims(64, s == 0);
     o->per_cu[4][s] = stream_blocks_dims(256, s == 0);
-    o->per_cu[5][s] = stream_blocks_f32(64, s == 0);
-    o->per_cu[6][s] = stream_blocks_f32(128, s == 0);
+    o->per_cu[5][s] = stream_blocks_f32(64, s == 0, false);
+    o->per_cu[6][s] = stream_blocks_f32(128, s == 0, false);
+    o->per_cu[7][s] = stream_blocks_f32(64, s == 0, true);
   }
 }
 
 }  // namespace
 
-int decode_stream_waves(int dtype, int head_dim, int stages, int group) {
+int decode_stream_waves(int dtype, int head_dim, int stages, int group, bool fine) {
   const bool f32 = dtype == kF32;
   const int sm = group <= 4 ? 0 : 1;
   const bool ring = !f32 && head_dim == 128;  // the variants with a tunable ring depth
   const int ns = ring && stages >= 2 && stages <= 4 ? stages : 2;
-  const int v = ring ? ns - 2 : f32 ? (head_dim == 64 ? 5 : 6) : (head_dim == 64 ? 3 : 4);
+  const int v = fine ? 7 : ring ? ns - 2 : f32 ? (head_dim == 64 ? 5 : 6) : (head_dim == 64 ? 3 : 4);
   int per_cu = 0, cus = 0;
   int dev = 0;
   if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) {
@@ -81,10 +83,12 @@ int decode_stream_waves(int dtype, int head_dim, int stages, int group) {
   if (per_cu <= 0) {
     using stream::StreamGeo;
     const int qr = sm == 0 ? 4 : 16;
-    const int slot = f32 ? (head_dim == 64 ? StreamGeo<float, 64>::slot_bytes(qr) : StreamGeo<float, 128>::slot_bytes(qr))
-                         : head_dim == 64    ? StreamGeo<bf16_t, 64>::slot_bytes(qr)
-                           : head_dim == 128 ? StreamGeo<bf16_t, 128>::slot_bytes(qr)
-                                             : StreamGeo<bf16_t, 256>::slot_bytes(qr);
+    const int slot = fine                ? StreamGeo<float, 64, true>::slot_bytes(qr)
+                     : f32 && head_dim == 64 ? StreamGeo<float, 64>::slot_bytes(qr)
+                     : f32               ? StreamGeo<float, 128>::slot_bytes(qr)
+                     : head_dim == 64    ? StreamGeo<bf16_t, 64>::slot_bytes(qr)
+                     : head_dim == 128   ? StreamGeo<bf16_t, 128>::slot_bytes(qr)
+                                         : StreamGeo<bf16_t, 256>::slot_bytes(qr);
     per_cu = 160 * 1024 / (ns * slot);
   }
   return cus * (per_cu > 1 ? per_cu : 1);

@@ -67,13 +67,14 @@
 namespace pf {
 namespace stream {
 
-// Geometry of a stage for rows of D elements of T.
-template <typename T, int D>
+// Geometry of a stage for rows of D elements of T. FINE: 16-key stages for
+// 256-byte rows too (DecodeParams::fine).
+template <typename T, int D, bool FINE = false>
 struct StreamGeo {
   static constexpr bool F32 = sizeof(T) == 4;
   static constexpr int RB = D * (int)sizeof(T);    // row bytes: 128, 256 or 512
   static constexpr int CPR = RB / 16;              // 16-byte chunks per row
-  static constexpr int SK = RB == 512 ? 16 : 32;   // keys per stage
+  static constexpr int SK = RB == 512 || FINE ? 16 : 32;  // keys per stage
   static constexpr int KPL = SK / 4;               // keys per lane (of its head)
   static constexpr int NU = SK / 16;               // 16-key tiles per stage
   static constexpr int TILE = SK * RB;             // one stage of K (or V)
@@ -408,10 +409,10 @@ __device__ inline int64_t wave_plan(const DecodeParams& p, int J, int W, int w, 
 // (short sequences, few of them): a workgroup per sequence, its four waves
 // taking a quarter of the stages each and merging through LDS at the end, so
 // no piece leaves the workgroup and no second kernel runs.
-template <typename T, int D, int PG, int NS, int QR, int NWV = 1>
+template <typename T, int D, int PG, int NS, int QR, int NWV = 1, bool FINE = false>
 __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams p) {
   using MF = Mfma16<T>;
-  using G = StreamGeo<T, D>;
+  using G = StreamGeo<T, D, FINE>;
   constexpr int SK = G::SK, RB = G::RB, KPL = G::KPL, NU = G::NU, NL = G::NL, RPL = G::RPL;
   constexpr int NSTEP = G::CPR / 4;  // K/Q chunk steps: lane group h reads chunk 4s + h
   constexpr int kSlotB = G::slot_bytes(QR);
@@ -880,9 +881,9 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
 // reading piece after piece took 30 us for 47 pieces of each of 32 heads (one
 // sequence of 1500 keys, 8 kv heads); 8 waves a head take 5 us. At 8-9 pieces
 // (B=16, 4096 keys): 7.5 -> 4.8 us.
-template <typename T, int D, int PG, int QR, int WPB>
+template <typename T, int D, int PG, int QR, int WPB, bool FINE>
 __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_combine_kernel(DecodeParams p) {
-  constexpr int SK = StreamGeo<T, D>::SK;
+  constexpr int SK = StreamGeo<T, D, FINE>::SK;
   constexpr int PER = D / 64;  // columns per lane
   constexpr int NB = 8;        // pieces in flight
   typedef float vp __attribute__((ext_vector_type(PER)));
@@ -1012,18 +1013,18 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
 // Waves per (b, h) of the combine: its pieces, about n_waves / sequences (and
 // at most one per stage), decide. Few pieces: a wave each, four (b, h) to a
 // workgroup; more: 4 or 8 waves share them.
-template <typename T, int D, int PG, int QR>
+template <typename T, int D, int PG, int QR, bool FINE>
 hipError_t launch_combine(const DecodeParams& p, hipStream_t st) {
   const int64_t n_bh = (int64_t)p.B * p.Hq;
   const int64_t seqs = (int64_t)p.B * p.Hkv * ((p.Hq / p.Hkv + 15) / 16);
   const int64_t len = PG <= 1 ? p.cache_len : (int64_t)p.pages_per_seq * p.page_size;
-  const int64_t pieces = std::min((int64_t)p.n_waves / seqs, len / StreamGeo<T, D>::SK) + 1;
+  const int64_t pieces = std::min((int64_t)p.n_waves / seqs, len / StreamGeo<T, D, FINE>::SK) + 1;
   if (pieces > 32)
-    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 8>), dim3((unsigned)n_bh), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 8, FINE>), dim3((unsigned)n_bh), dim3(512), 0, st, p);
   else if (pieces > 6)
-    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 4>), dim3((unsigned)n_bh), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 4, FINE>), dim3((unsigned)n_bh), dim3(256), 0, st, p);
   else
-    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 1>), dim3((unsigned)((n_bh + 3) / 4)),
+    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 1, FINE>), dim3((unsigned)((n_bh + 3) / 4)),
                        dim3(256), 0, st, p);
   return hipGetLastError();
 }
@@ -1043,9 +1044,9 @@ bool short_form(const DecodeParams& p) {
   return per_cu > 0 && !p.fixed_grid && p.stages == 2 && seqs <= 256 * per_cu && len <= kShortStages * G::SK;
 }
 
-template <typename T, int D, int PG, int NS, int QR>
+template <typename T, int D, int PG, int NS, int QR, bool FINE>
 hipError_t launch_stream(const DecodeParams& p, hipStream_t st) {
-  if constexpr (NS == 2 && kShortWaves * 2 * StreamGeo<T, D>::slot_bytes(QR) <= 160 * 1024) {
+  if constexpr (!FINE && NS == 2 && kShortWaves * 2 * StreamGeo<T, D>::slot_bytes(QR) <= 160 * 1024) {
     if (short_form<T, D, PG, QR>(p)) {
       const unsigned seqs = (unsigned)(p.B * p.Hkv * ((p.Hq / p.Hkv + 15) / 16));
       hipLaunchKernelGGL((pf_decode_stream_kernel<T, D, PG, 2, QR, kShortWaves>), dim3(seqs), dim3(64 * kShortWaves),
@@ -1053,26 +1054,27 @@ hipError_t launch_stream(const DecodeParams& p, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((pf_decode_stream_kernel<T, D, PG, NS, QR>), dim3((unsigned)p.n_waves), dim3(64), 0, st, p);
+  hipLaunchKernelGGL((pf_decode_stream_kernel<T, D, PG, NS, QR, 1, FINE>), dim3((unsigned)p.n_waves), dim3(64), 0, st,
+                     p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_combine<T, D, PG, QR>(p, st);
+  return launch_combine<T, D, PG, QR, FINE>(p, st);
 }
 
 // The ring depth is a tuning of the 16-bit head_dim 128 kernels; the others
 // run two stages.
-template <typename T, int D, int PG, int QR>
+template <typename T, int D, int PG, int QR, bool FINE>
 hipError_t launch_ns(const DecodeParams& p, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && D == 128) {
-    if (p.stages == 3) return launch_stream<T, D, PG, 3, QR>(p, st);
-    if (p.stages == 4) return launch_stream<T, D, PG, 4, QR>(p, st);
+    if (p.stages == 3) return launch_stream<T, D, PG, 3, QR, FINE>(p, st);
+    if (p.stages == 4) return launch_stream<T, D, PG, 4, QR, FINE>(p, st);
   }
-  return launch_stream<T, D, PG, 2, QR>(p, st);
+  return launch_stream<T, D, PG, 2, QR, FINE>(p, st);
 }
 
-template <typename T, int D, int PG>
+template <typename T, int D, int PG, bool FINE = false>
 hipError_t launch_qr(const DecodeParams& p, hipStream_t st) {
-  return (p.Hq / p.Hkv <= 4) ? launch_ns<T, D, PG, 4>(p, st) : launch_ns<T, D, PG, 16>(p, st);
+  return (p.Hq / p.Hkv <= 4) ? launch_ns<T, D, PG, 4, FINE>(p, st) : launch_ns<T, D, PG, 16, FINE>(p, st);
 }
 
 // Page groups: as many rows as one table lookup can serve (up to a stage).
@@ -1080,6 +1082,12 @@ hipError_t launch_qr(const DecodeParams& p, hipStream_t st) {
 template <typename T, int D>
 hipError_t launch_pg(const DecodeParams& p, bool paged, hipStream_t st) {
   using G = StreamGeo<T, D>;
+  if constexpr (sizeof(T) == 4 && D == 64) {
+    if (p.fine) {
+      if (!paged) return launch_qr<T, D, 0, true>(p, st);
+      return p.page_size % 16 == 0 ? launch_qr<T, D, 16, true>(p, st) : launch_qr<T, D, 4, true>(p, st);
+    }
+  }
   if (!paged) {
     if constexpr (sizeof(T) == 2 && D == 128) {
       if (p.positions != nullptr) return launch_qr<T, D, 1>(p, st);
@@ -1095,10 +1103,11 @@ hipError_t launch_pg(const DecodeParams& p, bool paged, hipStream_t st) {
 
 // Resident one-wave workgroups per CU (LDS-limited) of the kernel with `qr`
 // query rows and an `ns`-stage ring, 0 if the query fails.
-template <typename T, int D, int NS, int QR>
+template <typename T, int D, int NS, int QR, bool FINE = false>
 int blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pf_decode_stream_kernel<T, D, 0, NS, QR>, 64, 0) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pf_decode_stream_kernel<T, D, 0, NS, QR, 1, FINE>, 64, 0) !=
+      hipSuccess)
     return 0;
   return n;
 }

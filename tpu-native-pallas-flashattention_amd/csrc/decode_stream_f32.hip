@@ -3,7 +3,8 @@
 
 namespace pf {
 
-int stream_blocks_f32(int head_dim, bool small) {
+int stream_blocks_f32(int head_dim, bool small, bool fine) {
+  if (fine) return small ? stream::blocks_per_cu<float, 64, 2, 4, true>() : stream::blocks_per_cu<float, 64, 2, 16, true>();
   if (head_dim == 64)
     return small ? stream::blocks_per_cu<float, 64, 2, 4>() : stream::blocks_per_cu<float, 64, 2, 16>();
   return small ? stream::blocks_per_cu<float, 128, 2, 4>() : stream::blocks_per_cu<float, 128, 2, 16>();

@@ -285,8 +285,10 @@ struct DecodeParams {
   int stages;         // streaming kernel: LDS ring depth (2..4)
   int g;              // query heads per kv head (streaming kernel)
   int64_t part_q, part_rem;  // contiguous cache: the stages of the call divided by n_waves
+  int fine;           // 16-key stages (float32 head_dim 64)
   int fixed_grid;     // n_waves was set by hand (tuning): keep the persistent grid
   int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
+  int slot_waves;     // waves that the partial slots are sized for, at least n_waves
   // Fused decode step (streaming kernel, positions != null): the new token of
   // batch b is at pos = positions[b * pos_stride]; its k (rotated with table
   // row pos) and v go to cache slot pos (ring: pos % cache_size) and it
@@ -313,7 +315,7 @@ hipError_t launch_decode_combine(const DecodeParams& p, int dtype, bool paged, h
 // group: query heads per kv head
 bool decode_stream_supported(int dtype, int head_dim, int group, bool paged, int page_size);
 // resident one-wave workgroups on this device
-int decode_stream_waves(int dtype, int head_dim, int stages, int group);
+int decode_stream_waves(int dtype, int head_dim, int stages, int group, bool fine);
 int decode_stream_qrows(int group);               // query rows per partial slot
 hipError_t launch_decode_stream(const DecodeParams& p, int dtype, bool paged, hipStream_t stream);
 
