@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import check_fwd, check_grad, dev, host, note, qkv
+from gpu_util import TORCH_DT, check_fwd, check_grad, dev, host, note, qkv
 from oracle import attention_bwd_ref, attention_ref, rope_attention_ref
 from pallas_flash import _lib, flash_attention, flash_attention_rope, flash_attention_with_lse, precompute_rope
 
@@ -34,7 +34,7 @@ SHAPES = [  # B, Hq, Hkv, Sq, Sk, kv_len, causal
 
 
 def _args(dt, B, Hq, Hkv, Sq, Sk, kv_len, causal, D):
-    tag = _lib.PF_DTYPE[{"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dt]]
+    tag = _lib.PF_DTYPE[TORCH_DT[dt]]
     tail = (B, Hq, Hkv, Sq, Sk, D, kv_len, int(causal), 0.1, tag)
     return _lib.FwdArgs(8, 8, 8, 8, 8, *tail), _lib.BwdArgs(*[8] * 10, *tail)
 
@@ -91,6 +91,41 @@ def test_chunk_of_minus_infinity_scores():
     out = flash_attention(q, k, v)
     want = flash_attention(q, k, v, kv_len=512)
     check_fwd(host(out), host(want), "f32")
+
+
+@pytest.mark.parametrize("dt,D", [("f32", 64), ("f32", 128), ("bf16", 128)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_minus_infinity_rows_do_not_depend_on_the_split(dt, D, causal):
+    """Rows whose scores are -inf throughout, over the first block of keys, or
+    over later ones give what whole work items give: NaN for the first two
+    (the running max starts at -inf), the finite scores' result for the last."""
+    note(f"split: -inf rows {dt} D={D} causal={causal}")
+    S = 2048
+    fwd = _args(dt, 1, 1, 1, S, S, S, causal, D)[0]
+    L = _lib.lib()
+    ws_bytes = L.pf_attn_fwd_workspace_size(fwd)
+    assert ws_bytes > 0
+    g = torch.Generator("cuda").manual_seed(4)
+    q, k, v = (torch.randn((1, 1, S, D), device="cuda", generator=g).to(TORCH_DT[dt]) for _ in range(3))
+    q[0, 0, :, 0] = 1.0  # every row meets column 0 of K, -inf for some keys
+    for lo, hi, nan_rows in ((0, S, slice(0, S)), (0, 64, slice(0, S)), (64, S, slice(0, 0)), (600, 1400, slice(0, 0))):
+        k2 = k.clone()
+        k2[0, 0, lo:hi, 0] = -float("inf")
+        o, lse = [], []
+        for split in (False, True):
+            o.append(torch.empty_like(q))
+            lse.append(torch.empty((1, 1, S), dtype=torch.float32, device="cuda"))
+            a = _lib.FwdArgs(q.data_ptr(), k2.data_ptr(), v.data_ptr(), o[-1].data_ptr(), lse[-1].data_ptr(), 1, 1, 1,
+                             S, S, D, S, int(causal), 0.1, _lib.dtype_tag(q))
+            st = torch.cuda.current_stream().cuda_stream
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device="cuda")
+            assert (L.pf_attn_fwd_ws(a, ws.data_ptr(), ws_bytes, st) if split else L.pf_attn_fwd(a, st)) == 0
+        torch.cuda.synchronize()
+        for whole, cut in (o, lse):
+            assert torch.equal(torch.isnan(whole), torch.isnan(cut)), (lo, hi)
+        assert torch.isnan(o[0][0, 0, nan_rows]).all() and torch.isnan(o[0]).any() == (nan_rows.stop > 0)
+        if nan_rows.stop == 0:
+            check_fwd(host(o[1]), host(o[0]), dt)
 
 
 @pytest.mark.parametrize("B,H,S", [(8, 12, 1000), (5, 13, 1100), (3, 11, 1025)])

@@ -269,9 +269,12 @@ __global__ __launch_bounds__(256, (kFwdWgPerCu<T, D>)) void pf_attn_fwd_kernel(F
   }
 
 
-  // Running max, log2 domain (identical in both halves). Split: a chunk whose
-  // scores are all -inf must leave an empty partial (sum 0), not exp2(-inf + inf).
-  float m_run = SPLIT ? -__FLT_MAX__ : kNegInf;
+  // Running max, log2 domain (identical in both halves). From -inf, a row whose
+  // first block of scores is all -inf becomes NaN (exp2(-inf + inf)), as a row
+  // without a finite score has to; -inf scores further on drop out. So a split
+  // row's first chunk starts there too, and the later ones, which are "further
+  // on", start at the lowest finite value: all -inf, they leave sum 0.
+  float m_run = SPLIT && split > 0 ? -__FLT_MAX__ : kNegInf;
   float l_run = 0.f;      // running sum over this lane half's keys
   f32x16 acc[NDT];
 #pragma unroll
