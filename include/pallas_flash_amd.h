@@ -224,7 +224,10 @@ int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspa
  *   the generic kernel (computing at 64, 128 or 256 with the missing columns
  *   as zeros), with the same results to rounding.
  * workspace: at least pf_attn_decode_workspace_size(args) bytes, 256-byte
- * aligned device memory (contents on entry do not matter).
+ * aligned device memory (contents on entry do not matter). The size does not
+ * depend on cache_len or on the pointers (which may be NULL in the query): ask
+ * once for a cache and keep the workspace while it fills. For bf16/f16 with
+ * head_dim 128 it is the same for every batch and cache_size, too.
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* q;
@@ -257,7 +260,8 @@ int pf_attn_decode(const pf_attn_decode_args* args, void* stream);
  * streaming kernel takes page sizes that are a multiple of 4 (of 8 for bf16/f16
  * at head_dim 64), so that a load stays inside one page, the generic split-KV
  * kernel the others, with the same results to rounding.
- * workspace: at least pf_paged_attn_workspace_size(args) bytes.
+ * workspace: at least pf_paged_attn_workspace_size(args) bytes; the size does
+ * not depend on the context lengths or the pointers.
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* q;
@@ -286,13 +290,13 @@ int pf_paged_attn(const pf_paged_attn_args* args, void* stream);
  * ignored. The split-KV partials go to a static device array of
  * PF_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
  * process ends.
- *  - A call whose partials need more than PF_NOALLOC_SCRATCH_BYTES
- *    (pf_paged_attn_workspace_size(args) larger) returns PF_ERR_WORKSPACE
- *    and enqueues nothing. The streaming kernel (pf_paged_attn) needs at most
- *    about 16.5 MiB (bf16/f16 head_dim 256 with more than 4 heads per KV head:
- *    24.2 MiB) at the default tuning on a 256-CU device, whatever the batch; the
- *    generic kernel needs about
- *    batch * num_heads * splits * 520 bytes.
+ *  - A call whose partials need more than PF_NOALLOC_SCRATCH_BYTES returns
+ *    PF_ERR_WORKSPACE and enqueues nothing (the partials of the kernel that it
+ *    runs; pf_paged_attn_workspace_size(args) can be larger). The streaming
+ *    kernel (pf_paged_attn) needs at most about 16.5 MiB (bf16/f16 head_dim 256
+ *    with more than 4 heads per KV head: 24.2 MiB) at the default tuning on a
+ *    256-CU device, whatever the batch; the generic kernel needs about
+ *    batch * num_heads * splits * (4 * head_dim + 8) bytes.
  *  - A call uses the array of the device `stream` belongs to (the null
  *    stream's: the current device).
  *  - Every call on one GPU shares that GPU's array: calls that overlap on

@@ -164,6 +164,28 @@ def test_decode_workspace_of_a_longer_cache_serves_a_shorter_one(L, heads, kv):
     assert ws == sorted(ws) and ws[0] > 0
 
 
+NULLS = dict(q=None, k_cache=None, v_cache=None)
+ALIGNED = dict(q=256, k_cache=512, v_cache=1024)
+UNALIGNED = dict(q=256, k_cache=514, v_cache=1026)
+
+
+@pytest.mark.parametrize("dtype,D", [(1, 128), (2, 128), (1, 64), (2, 256), (0, 64), (0, 128), (1, 96)])
+@pytest.mark.parametrize("heads,kv", [(32, 8), (32, 2), (40, 1)])
+def test_decode_workspace_depends_on_the_shape_alone(L, dtype, D, heads, kv):
+    """One query serves a cache while it fills, wherever the operands lie;
+    16-bit head_dim 128: any batch and cache as well."""
+    base = dict(dtype=dtype, head_dim=D, num_heads=heads, num_kv_heads=kv)
+    sizes = {L.pf_attn_decode_workspace_size(_dec(cache_len=n, **p, **base))
+             for n in (1, 63, 300, 1537, 4001, 6000, 8192) for p in (NULLS, ALIGNED, UNALIGNED)}
+    assert len(sizes) == 1 and min(sizes) > 0
+    paged = {L.pf_paged_attn_workspace_size(_paged(k_pages=p["k_cache"], v_pages=p["v_cache"], q=p["q"], **base))
+             for p in (NULLS, ALIGNED, UNALIGNED)}
+    assert len(paged) == 1 and min(paged) > 0
+    if D == 128 and dtype != 0:
+        for other in (dict(batch=1), dict(batch=4096), dict(batch=1, cache_size=7, cache_len=7)):
+            assert {L.pf_attn_decode_workspace_size(_dec(**{**base, **other}))} == sizes == paged
+
+
 def _paged(**over):
     base = dict(q=8, k_pages=8, v_pages=8, block_tables=8, context_lens=8, o=8, batch=128,
                 num_heads=32, num_kv_heads=8, num_pages=16384, page_size=64, head_dim=128,

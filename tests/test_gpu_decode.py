@@ -13,7 +13,7 @@ import torch
 
 from gpu_util import check_fwd, dev, host, max_abs, note
 from oracle import decode_ref
-from pallas_flash import flash_attention, flash_attention_decode
+from pallas_flash import _lib, flash_attention, flash_attention_decode
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +101,32 @@ def test_ring_layout_is_permutation_invariant(dt):
                                              dev(np.roll(v, shift, axis=2), dt), capacity))
         assert max_abs(in_order, rolled) < (2e-3 if dt == "f32" else 2e-2)
     check_fwd(in_order, decode_ref(host(dev(q, dt)), host(dev(k, dt)), host(dev(v, dt)), capacity), dt)
+
+
+@pytest.mark.parametrize("dt,D,skew", [("bf16", 128, 0), ("f32", 128, 1), ("f16", 64, 1), ("bf16", 256, 1),
+                                       ("f32", 64, 0)])
+def test_workspace_asked_for_once_serves_the_growing_cache(dt, D, skew):
+    """The size asked for at the first token, with no pointers yet, holds for
+    every later length; skew: for a cache between two 16-byte boundaries too."""
+    note(f"decode workspace {dt} D={D} skew={skew}")
+    rng = np.random.default_rng(D)
+    B, Hq, Hkv, cap = 8, 8, 2, 6000
+    q = dev(rng.standard_normal((B, Hq, 1, D)), dt)
+    caches = []
+    for _ in range(2):
+        gen = torch.Generator("cuda").manual_seed(D + len(caches))
+        flat = torch.randn(B * Hkv * cap * D + 8, device="cuda", generator=gen).to(q.dtype)
+        caches.append(flat[skew:skew + B * Hkv * cap * D].view(B, Hkv, cap, D))
+    L = _lib.lib()
+    o = torch.empty_like(q)
+
+    def args(length, ptrs, ws=None, n=0):
+        return _lib.DecodeArgs(*ptrs, B, Hq, Hkv, cap, D, length, D ** -0.5, _lib.dtype_tag(q), ws, n)
+
+    n = L.pf_attn_decode_workspace_size(args(1, (None,) * 4))
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    ptrs = (q.data_ptr(), caches[0].data_ptr(), caches[1].data_ptr(), o.data_ptr())
+    for length in (1, 700, 3001, cap):
+        st = L.pf_attn_decode(args(length, ptrs, ws.data_ptr(), n), torch.cuda.current_stream().cuda_stream)
+        assert st == _lib.PF_OK, length
+        check_fwd(host(o), decode_ref(host(q), host(caches[0]), host(caches[1]), length), dt)

@@ -24,7 +24,7 @@ import numpy as np
 import pytest
 import torch
 
-from gpu_util import dev, note
+from gpu_util import check_fwd, dev, host, note
 from pallas_flash import _lib
 
 pytestmark = pytest.mark.gpu
@@ -114,6 +114,22 @@ def test_noalloc_refuses_partials_past_the_array():
     assert st == _lib.PF_ERR_WORKSPACE
     torch.cuda.synchronize()
     assert bool((o == 3.0).all())
+
+
+def test_noalloc_takes_a_grid_set_by_hand_past_the_array():
+    """More waves than the array holds partials for (decode_waves, head_dim 256,
+    16 heads per KV head): the generic kernel, whose partials fit, answers."""
+    note("noalloc: hand-set grid past the array")
+    L = _lib.lib()
+    q, kp, vp, tt, tl = _problem(60, 12, 32, 2, 16, 176, 12 * 176, "bf16", 176 * 16, 256)
+    want, got = torch.full_like(q, float("nan")), torch.full_like(q, float("nan"))
+    _with_workspace(L, _args(q, kp, vp, tt, tl, want), q)
+    with _lib.tuning(decode_waves=4096):
+        st = L.pf_paged_attn_noalloc(ctypes.byref(_args(q, kp, vp, tt, tl, got)),
+                                     torch.cuda.current_stream().cuda_stream)
+    assert st == _lib.PF_OK, st
+    torch.cuda.synchronize()
+    check_fwd(host(got), host(want), "bf16")  # another kernel: equal to rounding
 
 
 def _graph_check(capture_first: bool) -> None:

@@ -3,6 +3,7 @@
 // (no HIP call before validation passes), fills a kernel parameter block and
 // enqueues on the caller's stream. Nothing here allocates or synchronises.
 #include <math.h>
+#include <stdint.h>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -550,13 +551,17 @@ static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Key-chunk size for split-KV: enough (b, kv head, chunk) waves to fill the
 // chip several times over (256 CUs x 8 resident waves), chunks a multiple of
 // the 64-key block and at least 256 keys so each wave streams a useful run.
-static int decode_chunk(int64_t units, int max_len) {
+constexpr int kMinChunk = 256;
+static int64_t decode_splits(int64_t units) {  // the chunks aimed at
   const int64_t target_waves = 4096;
-  int64_t n_split = (target_waves + units - 1) / (units > 0 ? units : 1);
-  if (n_split < 1) n_split = 1;
+  const int64_t n = (target_waves + units - 1) / (units > 0 ? units : 1);
+  return n > 1 ? n : 1;
+}
+static int decode_chunk(int64_t units, int max_len) {
+  const int64_t n_split = decode_splits(units);
   int64_t chunk = (max_len + n_split - 1) / n_split;
   chunk = ((chunk + 63) / 64) * 64;
-  if (chunk < 256) chunk = 256;
+  if (chunk < kMinChunk) chunk = kMinChunk;
   return (int)chunk;
 }
 
@@ -567,17 +572,19 @@ static int decode_chunk(int64_t units, int max_len) {
 // of the 16-bit head_dim 128 kernels) and decode_waves (grid size; any value
 // >= 1 is correct, only the resident count is fast).
 // A short problem starts only as many waves as it has stages (32 keys; 16 in
-// float32 at head_dim 128 and with fine stages), and keeps no partial slots for more; at 16-bit
-// head_dim 256 a wave takes at least two 16-key stages, which halves the slots
-// for 0.6 us. One stage a wave also cuts equal sequences alike, whatever
-// their place in the list. max_len: the most keys a sequence can have.
+// float32 at head_dim 128 and with fine stages); at 16-bit head_dim 256 a wave
+// takes at least two 16-key stages, which halves the pieces to merge for 0.6 us.
+// One stage a wave also cuts equal sequences alike, whatever their place in the
+// list. max_len: the most keys a sequence can have.
+static int stream_grid(int dtype, int32_t head_dim, int group, bool fine) {
+  const int wv = tuning().decode_waves.load(std::memory_order_relaxed);
+  if (wv > 0) return wv;
+  return pf::decode_stream_waves(dtype, head_dim, tuning().decode_stages.load(std::memory_order_relaxed), group, fine);
+}
 static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
-  Tuning& t = tuning();
-  const int ns = t.decode_stages.load(std::memory_order_relaxed);
-  p->stages = ns;
-  const int wv = t.decode_waves.load(std::memory_order_relaxed);
   const int group = p->Hq / p->Hkv;
-  p->fixed_grid = wv > 0;
+  p->stages = tuning().decode_stages.load(std::memory_order_relaxed);
+  p->fixed_grid = tuning().decode_waves.load(std::memory_order_relaxed) > 0;
   // Float32 at head_dim 64: a stage is 0.9 us of float32 MFMAs, so with a few
   // stages a wave half as long ones, on twice as many waves (8 a CU), divide
   // more evenly and hide each other's loads: 16 x 4 sequences of 64-2048 keys
@@ -591,15 +598,10 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   const bool f32 = dtype == PF_DTYPE_F32, can_fine = f32 && p->D == 64;
   p->fine = can_fine && max_len > 12 * 32 && stages32 > 4 * kCus && stages32 <= 32 * 4 * kCus;
   const int sk = p->D * (f32 ? 4 : 2) == 512 || p->fine ? 16 : 32;  // keys per stage
-  auto waves = [&](bool fine, int unit) {
-    const int64_t runs = seqs * ((max_len + unit - 1) / unit);
-    const int n = wv > 0 ? wv : pf::decode_stream_waves(dtype, p->D, ns, group, fine);
-    return n > runs ? (int)(runs > 1 ? runs : 1) : n;
-  };
-  p->n_waves = waves(p->fine != 0, f32 ? sk : 32);
-  // Partials are sized for either choice, so that a workspace made for a long
-  // cache also serves a shorter one.
-  p->slot_waves = can_fine ? std::max(p->n_waves, waves(true, 16)) : p->n_waves;
+  const int unit = f32 ? sk : 32;
+  const int64_t runs = seqs * ((max_len + unit - 1) / unit);
+  const int grid = stream_grid(dtype, p->D, group, p->fine != 0);
+  p->n_waves = grid > runs ? (int)(runs > 1 ? runs : 1) : grid;
   p->n_split = 0;
   p->chunk = 0;
   p->g = group;
@@ -624,7 +626,8 @@ static bool stream_aligned(const void* q, const void* k, const void* v) {
 // fall back to the generic kernel past its range and for unaligned operands.
 static bool stream_only(int32_t head_dim, int32_t dtype) { return head_dim == 128 && dtype != PF_DTYPE_F32; }
 
-static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
+// *streams: whether the call's shape is one of the streaming kernel's.
+static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p, bool* streams) {
   if (!a) return PF_ERR_INVALID;
   if (a->batch < 0 || a->num_heads < 1 || a->num_kv_heads < 1 || a->cache_size < 1)
     return PF_ERR_INVALID;
@@ -648,10 +651,11 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   p->cache_size = a->cache_size;
   p->cache_len = a->cache_len;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
+  *streams = false;
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, false, 0)) {
     // buffer offsets within one (b, kv head) run are 32-bit
-    if (stream_range_ok(a->cache_size, a->head_dim, a->dtype) &&
-        (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_cache, a->v_cache))) {
+    *streams = stream_range_ok(a->cache_size, a->head_dim, a->dtype);
+    if (*streams && (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_cache, a->v_cache))) {
       if (stream_setup(p, a->dtype, a->cache_len) <= 0) return PF_ERR_LAUNCH;
       return PF_OK;
     }
@@ -663,24 +667,53 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p) {
   return PF_OK;
 }
 
-// Partial slots: streaming kernel one per piece (piece_slot) x query rows;
-// generic kernel one per (b, query head, chunk).
+// The bytes of `slots` partials (max, sum and D accumulators each).
+static size_t partial_bytes(size_t slots, int D) {
+  return align256(slots * D * sizeof(float)) + align256(slots * 2 * sizeof(float));
+}
+
+// Partial slots of a launch: streaming kernel one per piece (piece_slot) x
+// query rows -- at most one piece that a wave opens with and one that it ends
+// with --, generic kernel one per (b, query head, chunk).
 static size_t decode_slots(const pf::DecodeParams& p) {
-  if (p.n_waves > 0) {
-    const int group = p.Hq / p.Hkv;
-    const int64_t seqs = (int64_t)p.B * p.Hkv * ((group + 15) / 16);
-    return (size_t)(p.slot_waves + (seqs < p.slot_waves ? seqs : p.slot_waves)) * pf::decode_stream_qrows(group);
+  if (p.n_waves == 0) return (size_t)p.B * p.Hq * p.n_split;
+  const int group = p.Hq / p.Hkv;
+  const int64_t seqs = (int64_t)p.B * p.Hkv * ((group + 15) / 16);
+  return (size_t)(p.n_waves + (seqs < p.n_waves ? seqs : p.n_waves)) * pf::decode_stream_qrows(group);
+}
+
+// What the size queries answer: enough for the same call with any cache length
+// up to `cap` keys and wherever its operands lie, and for the streaming forms
+// whatever the batch -- a program asks once and keeps the workspace while its
+// sequences grow. So it counts two pieces for every wave of a full streaming
+// grid, and the generic kernel's chunks where a call can end up there.
+static size_t decode_ws_most(const pf::DecodeParams& p, int dtype, bool streams, int64_t cap) {
+  const int group = p.Hq / p.Hkv;
+  size_t most = 0;
+  if (streams) {
+    int waves = stream_grid(dtype, p.D, group, false);
+    if (dtype == PF_DTYPE_F32 && p.D == 64) waves = std::max(waves, stream_grid(dtype, p.D, group, true));
+    most = partial_bytes((size_t)2 * waves * pf::decode_stream_qrows(group), p.D);
+    if (stream_only(p.dr, dtype)) return most;
   }
-  return (size_t)p.B * p.Hq * p.n_split;
+  // decode_chunk's chunks have at least kMinChunk keys and at least cap / splits.
+  const int64_t units = (int64_t)p.B * p.Hkv * ((group + 31) / 32);
+  int64_t n = std::min(decode_splits(units), (cap + kMinChunk - 1) / kMinChunk);
+  if (n < 1) n = 1;
+  return std::max(most, partial_bytes((size_t)p.B * p.Hq * n, p.D));
 }
 
-static size_t decode_ws_bytes(const pf::DecodeParams& p) {
-  const size_t slots = decode_slots(p);
-  return align256(slots * p.D * sizeof(float)) + align256(slots * 2 * sizeof(float));
+// The bytes that a launch insists on: what it uses; the 16-bit head_dim 128
+// forms the full size that their query answers (or more, where another thread
+// has just lowered decode_waves).
+static size_t decode_ws_bytes(const pf::DecodeParams& p, int dtype) {
+  const size_t used = partial_bytes(decode_slots(p), p.D);
+  if (p.n_waves == 0 || !stream_only(p.dr, dtype)) return used;
+  return std::max(used, decode_ws_most(p, dtype, true, 0));
 }
 
-static int bind_workspace(pf::DecodeParams* p, void* ws, size_t bytes) {
-  const size_t need = decode_ws_bytes(*p);
+static int bind_workspace(pf::DecodeParams* p, int dtype, void* ws, size_t bytes) {
+  const size_t need = decode_ws_bytes(*p, dtype);
   if (need == 0) return PF_OK;
   if (!ws || bytes < need || ((uintptr_t)ws & 255) != 0) return PF_ERR_WORKSPACE;
   const size_t slots = decode_slots(*p);
@@ -691,22 +724,26 @@ static int bind_workspace(pf::DecodeParams* p, void* ws, size_t bytes) {
 
 size_t pf_attn_decode_workspace_size(const pf_attn_decode_args* a) {
   pf::DecodeParams p;
-  if (fill_decode(a, &p) != PF_OK) return 0;
-  return decode_ws_bytes(p);
+  bool streams;
+  if (fill_decode(a, &p, &streams) != PF_OK) return 0;
+  return decode_ws_most(p, a->dtype, streams, a->cache_size);
 }
 
 int pf_attn_decode(const pf_attn_decode_args* a, void* stream) {
   pf::DecodeParams p;
-  int st = fill_decode(a, &p);
+  bool streams;
+  int st = fill_decode(a, &p, &streams);
   if (st != PF_OK) return st;
   if (!a->q || !a->k_cache || !a->v_cache || !a->o) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  st = bind_workspace(&p, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
   return finish(pf::launch_decode(p, a->dtype, false, (hipStream_t)stream));
 }
 
-static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p) {
+// most_ws: the partials' room, where it cannot grow (the streaming grid can be
+// set by hand to more waves than fit; the generic kernel then runs).
+static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p, bool* streams, size_t most_ws) {
   if (!a) return PF_ERR_INVALID;
   // paged.py:129-149: Sq == 1 (implied by the struct), heads divisible, table [B, P], lens [B].
   if (a->batch < 0 || a->num_heads < 1 || a->num_kv_heads < 1 || a->num_pages < 1 ||
@@ -736,13 +773,16 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p) {
   p->page_size = a->page_size;
   p->pages_per_seq = a->pages_per_seq;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
+  *streams = false;
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, true, a->page_size)) {
-    if (stream_range_ok(a->page_size, a->head_dim, a->dtype) &&
-        (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_pages, a->v_pages))) {
+    const bool only = stream_only(a->head_dim, a->dtype);
+    *streams = stream_range_ok(a->page_size, a->head_dim, a->dtype);
+    if (*streams && (only || stream_aligned(a->q, a->k_pages, a->v_pages))) {
       if (stream_setup(p, a->dtype, max_len) <= 0) return PF_ERR_LAUNCH;
-      return PF_OK;
+      if (only || decode_ws_bytes(*p, a->dtype) <= most_ws) return PF_OK;
+      p->n_waves = 0;
     }
-    if (stream_only(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
+    if (only) return PF_ERR_UNSUPPORTED;
   }
   p->chunk = decode_chunk(units, (int)(max_len > 0 ? max_len : 1));
   p->n_split = max_len > 0 ? (int)((max_len + p->chunk - 1) / p->chunk) : 1;
@@ -752,18 +792,20 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p) {
 
 size_t pf_paged_attn_workspace_size(const pf_paged_attn_args* a) {
   pf::DecodeParams p;
-  if (fill_paged(a, &p) != PF_OK) return 0;
-  return decode_ws_bytes(p);
+  bool streams;
+  if (fill_paged(a, &p, &streams, SIZE_MAX) != PF_OK) return 0;
+  return decode_ws_most(p, a->dtype, streams, (int64_t)a->pages_per_seq * a->page_size);
 }
 
 int pf_paged_attn(const pf_paged_attn_args* a, void* stream) {
   pf::DecodeParams p;
-  int st = fill_paged(a, &p);
+  bool streams;
+  int st = fill_paged(a, &p, &streams, SIZE_MAX);
   if (st != PF_OK) return st;
   if (!a->q || !a->k_pages || !a->v_pages || !a->o || !a->context_lens) return PF_ERR_INVALID;
   if (a->pages_per_seq > 0 && !a->block_tables) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  st = bind_workspace(&p, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
   return finish(pf::launch_decode(p, a->dtype, true, (hipStream_t)stream));
 }
@@ -816,17 +858,17 @@ extern "C" {
 
 int pf_paged_attn_noalloc(const pf_paged_attn_args* a, void* stream) {
   pf::DecodeParams p;
-  int st = fill_paged(a, &p);
+  bool streams;
+  int st = fill_paged(a, &p, &streams, PF_NOALLOC_SCRATCH_BYTES);
   if (st != PF_OK) return st;
   if (!a->q || !a->k_pages || !a->v_pages || !a->o || !a->context_lens) return PF_ERR_INVALID;
   if (a->pages_per_seq > 0 && !a->block_tables) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  const size_t need = decode_ws_bytes(p);
-  if (need > (size_t)PF_NOALLOC_SCRATCH_BYTES) return PF_ERR_WORKSPACE;
+  if (decode_ws_bytes(p, a->dtype) > (size_t)PF_NOALLOC_SCRATCH_BYTES) return PF_ERR_WORKSPACE;
   void* ws = nullptr;
   st = scratch_address((hipStream_t)stream, &ws);
   if (st != PF_OK) return st;
-  st = bind_workspace(&p, ws, PF_NOALLOC_SCRATCH_BYTES);
+  st = bind_workspace(&p, a->dtype, ws, PF_NOALLOC_SCRATCH_BYTES);
   if (st != PF_OK) return st;
   return finish(pf::launch_decode(p, a->dtype, true, (hipStream_t)stream));
 }
@@ -923,7 +965,7 @@ static int fill_decode_step(const pf_attn_decode_step_args* a, pf::DecodeParams*
 size_t pf_attn_decode_step_workspace_size(const pf_attn_decode_step_args* a) {
   pf::DecodeParams p;
   if (fill_decode_step(a, &p) != PF_OK) return 0;
-  return decode_ws_bytes(p);
+  return decode_ws_bytes(p, a->dtype);
 }
 
 int pf_attn_decode_step(const pf_attn_decode_step_args* a, void* stream) {
@@ -933,7 +975,7 @@ int pf_attn_decode_step(const pf_attn_decode_step_args* a, void* stream) {
   if (a->batch == 0) return PF_OK;
   if (!a->q || !a->k_new || !a->v_new || !a->k_cache || !a->v_cache || !a->o || !a->positions)
     return PF_ERR_INVALID;
-  st = bind_workspace(&p, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
   return finish(pf::launch_decode(p, a->dtype, false, (hipStream_t)stream));
 }

@@ -288,7 +288,6 @@ struct DecodeParams {
   int fine;           // 16-key stages (float32 head_dim 64)
   int fixed_grid;     // n_waves was set by hand (tuning): keep the persistent grid
   int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
-  int slot_waves;     // waves that the partial slots are sized for, at least n_waves
   // Fused decode step (streaming kernel, positions != null): the new token of
   // batch b is at pos = positions[b * pos_stride]; its k (rotated with table
   // row pos) and v go to cache slot pos (ring: pos % cache_size) and it
