@@ -220,9 +220,10 @@ int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspa
  *   head_dim <= 256 (bf16/f16) or 128 (float32), a multiple of 8 (bf16/f16)
  *   or 4 (float32): rows are read in place; head_dim 64, 128 and (bf16/f16)
  *   256 run the streaming kernel -- off bf16/f16 head_dim 128, for groups of
- *   at most 16 query heads per KV head --, other head dims and larger groups
- *   the generic kernel (computing at 64, 128 or 256 with the missing columns
- *   as zeros), with the same results to rounding.
+ *   at most 16 query heads per KV head --, other head dims, larger groups and
+ *   operands that are not 16-byte aligned the generic kernel (computing at 64,
+ *   128 or 256 with the missing columns as zeros), with the same results to
+ *   rounding.
  * workspace: at least pf_attn_decode_workspace_size(args) bytes, 256-byte
  * aligned device memory (contents on entry do not matter). The size does not
  * depend on cache_len or on the pointers (which may be NULL in the query): ask
@@ -389,7 +390,8 @@ int pf_paged_cache_write(const pf_paged_cache_write_args* args, void* stream);
  *             (valid iff pos >= 0); model.py:475-476
  * With RoPE, a valid position is also < rope_len. An invalid position writes
  * nothing and gives o = 0 for that batch.
- * Supported: bf16 / f16 with head_dim 128 (PF_ERR_UNSUPPORTED otherwise).
+ * Supported: bf16 / f16 with head_dim 128 (PF_ERR_UNSUPPORTED otherwise); q,
+ * k_cache and v_cache 16-byte aligned (PF_ERR_INVALID otherwise).
  * workspace: at least pf_attn_decode_step_workspace_size(args) bytes,
  * 256-byte aligned (contents on entry do not matter).
  * ------------------------------------------------------------------------- */

@@ -20,7 +20,8 @@ import torch
 
 from gpu_util import check_fwd, dev, host, note
 from oracle import decode_ref, paged_ref
-from pallas_flash import _lib, flash_attention_decode, paged_flash_attention
+from pallas_flash import (_lib, flash_attention_decode, flash_attention_decode_step, paged_flash_attention,
+                          precompute_rope)
 
 pytestmark = pytest.mark.gpu
 
@@ -128,7 +129,7 @@ def test_f32_fine_stages_paged(Hq, page):
     assert (out[0] == 0).all()
 
 
-@pytest.mark.parametrize("dt,D", [("f16", 64), ("bf16", 256), ("f32", 128)])
+@pytest.mark.parametrize("dt,D", [("f16", 64), ("bf16", 256), ("f32", 128), ("bf16", 128)])
 def test_unaligned_cache_keeps_the_generic_kernel(dt, D):
     """A contiguous cache that starts between two 16-byte boundaries: the
     streaming kernel's loads want aligned rows, so the generic kernel reads it."""
@@ -146,3 +147,62 @@ def test_unaligned_cache_keeps_the_generic_kernel(dt, D):
         caches.append(view)
     out = host(flash_attention_decode(tq, *caches, L))
     check_fwd(out, decode_ref(host(tq), host(caches[0]), host(caches[1]), L), dt)
+
+
+def _skewed(x):
+    """x's values in a contiguous tensor that starts between two 16-byte boundaries."""
+    flat = torch.empty(x.numel() + 8, dtype=x.dtype, device="cuda")
+    view = flat[1:1 + x.numel()].view(x.shape)
+    view.copy_(x)
+    assert view.is_contiguous() and view.data_ptr() % 16 != 0
+    return view
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,w", [(3, 8, 2, 0), (11, 8, 2, 4), (5, 40, 2, 1)])
+@pytest.mark.parametrize("what", ["decode", "paged"])
+def test_unaligned_operands_at_16bit_head_dim_128(what, B, Hq, Hkv, w):
+    """The form whose workspace has one size: with a grid of a few waves (w) that
+    size holds the partials of a few batches, and the generic kernel runs
+    slice after slice (11 batches by 4; 5 by 1)."""
+    note(f"unaligned 16-bit head_dim 128 {what} B={B} Hq={Hq} w={w}")
+    rng = np.random.default_rng(B)
+    D, page, n = 128, 16, 60
+    tq = _skewed(dev(rng.standard_normal((B, Hq, 1, D)), "bf16"))
+    with _lib.tuning(decode_waves=w):
+        if what == "decode":
+            tk, tv = (_skewed(dev(rng.standard_normal((B, Hkv, page * n, D)), "bf16")) for _ in range(2))
+            out = host(flash_attention_decode(tq, tk, tv, 901))
+            want = decode_ref(host(tq), host(tk), host(tv), 901)
+        else:
+            tk, tv = (_skewed(dev(rng.standard_normal((B * n, Hkv, page, D)), "bf16")) for _ in range(2))
+            lens = rng.integers(0, page * n + 1, B).astype(np.int32)
+            table = rng.permutation(B * n).reshape(B, n).astype(np.int32)
+            out = host(paged_flash_attention(tq, tk, tv, torch.as_tensor(table), torch.as_tensor(lens)))
+            want = paged_ref(host(tq), host(tk), host(tv), table, lens)
+    check_fwd(out, want, "bf16")
+
+
+@pytest.mark.parametrize("skew", ["q", "k", "v", "all"])
+def test_unaligned_decode_step(skew):
+    """The fused step through the public call: as with aligned operands, the
+    caches written in place; the C entry refuses them."""
+    note(f"unaligned decode step {skew}")
+    rng = np.random.default_rng(7)
+    B, Hq, Hkv, C, D = 3, 8, 2, 500, 128
+    ops = [dev(rng.standard_normal(s), "bf16") for s in ((B, Hq, 1, D), (B, Hkv, C, D), (B, Hkv, C, D))]
+    k_new, v_new = (dev(rng.standard_normal((B, Hkv, 1, D)), "bf16") for _ in range(2))
+    cos, sin = (t.cuda() for t in precompute_rope(1200, D, 10000.0))
+    pos = torch.tensor([3, 499, 1150], dtype=torch.int32, device="cuda")
+    own = [_skewed(t) if skew in (name, "all") else t.clone() for name, t in zip("qkv", ops)]
+    ptrs = [t.data_ptr() for t in own]
+    got = flash_attention_decode_step(own[0], k_new, v_new, own[1], own[2], pos, cos, sin, ring=True)
+    want = flash_attention_decode_step(ops[0], k_new, v_new, ops[1], ops[2], pos, cos, sin, ring=True)
+    assert ptrs == [t.data_ptr() for t in own]
+    assert torch.equal(got, want) and torch.equal(own[1], ops[1]) and torch.equal(own[2], ops[2])
+    args = _lib.DecodeStepArgs(ptrs[0], k_new.data_ptr(), v_new.data_ptr(), ptrs[1], ptrs[2], got.data_ptr(),
+                               pos.data_ptr(), 1, None, None, 0, B, Hq, Hkv, C, D, 1, 0.1, _lib.dtype_tag(k_new),
+                               None, 0)
+    L = _lib.lib()
+    ws = torch.empty(L.pf_attn_decode_step_workspace_size(args), dtype=torch.uint8, device="cuda")
+    args.workspace, args.workspace_bytes = ws.data_ptr(), ws.numel()
+    assert L.pf_attn_decode_step(args, None) == _lib.PF_ERR_INVALID

@@ -622,9 +622,33 @@ static bool stream_range_ok(int64_t rows, int32_t head_dim, int32_t dtype) {
 static bool stream_aligned(const void* q, const void* k, const void* v) {
   return (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
 }
-// The 16-bit head_dim 128 forms run on the streaming kernel alone; the others
-// fall back to the generic kernel past its range and for unaligned operands.
+// Forms with one workspace size, whatever the batch and the cache; past the
+// streaming kernel's range they are refused, where the others run the generic
+// kernel. Unaligned operands run it in either case.
 static bool stream_only(int32_t head_dim, int32_t dtype) { return head_dim == 128 && dtype != PF_DTYPE_F32; }
+// Partial slots of that one size: two pieces for every wave of a full grid, and
+// at least a batch's heads, for the generic kernel.
+static int64_t stream_room(const pf::DecodeParams& p, int dtype) {
+  const int group = p.Hq / p.Hkv;
+  return std::max((int64_t)2 * stream_grid(dtype, p.D, group, false) * pf::decode_stream_qrows(group), (int64_t)p.Hq);
+}
+
+// The generic kernel's chunks of up to max_len keys. room > 0: no more partials
+// than that, by fewer chunks and, past one chunk, by batches (p->slice) whose
+// launches follow each other on the stream.
+static int generic_setup(pf::DecodeParams* p, int64_t max_len, int64_t room) {
+  const int64_t per_batch = (int64_t)p->Hkv * ((p->Hq / p->Hkv + 31) / 32);
+  p->n_waves = 0;
+  p->slice = p->B;
+  if (room > 0) p->slice = (int)std::min((int64_t)p->B, room / p->Hq);
+  p->chunk = decode_chunk(per_batch * p->slice, (int)max_len);
+  if (room > 0 && p->slice > 0) {
+    const int64_t n = room / ((int64_t)p->slice * p->Hq);
+    p->chunk = (int)std::max((int64_t)p->chunk, ((max_len + n - 1) / n + 63) / 64 * 64);
+  }
+  p->n_split = (int)((max_len + p->chunk - 1) / p->chunk);
+  return per_batch * p->slice * p->n_split > kMaxGrid ? PF_ERR_UNSUPPORTED : PF_OK;
+}
 
 // *streams: whether the call's shape is one of the streaming kernel's.
 static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p, bool* streams) {
@@ -637,7 +661,6 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p, bool* 
   if (!dtype_ok(a->dtype)) return PF_ERR_UNSUPPORTED;
   if (!decode_head_dim_ok(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
   const int g = a->num_heads / a->num_kv_heads;
-  const int64_t units = (int64_t)a->batch * a->num_kv_heads * ((g + 31) / 32);
   *p = pf::DecodeParams{};
   p->q = a->q;
   p->k = a->k_cache;
@@ -652,19 +675,15 @@ static int fill_decode(const pf_attn_decode_args* a, pf::DecodeParams* p, bool* 
   p->cache_len = a->cache_len;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
   *streams = false;
+  const bool only = stream_only(a->head_dim, a->dtype);
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, false, 0)) {
     // buffer offsets within one (b, kv head) run are 32-bit
     *streams = stream_range_ok(a->cache_size, a->head_dim, a->dtype);
-    if (*streams && (stream_only(a->head_dim, a->dtype) || stream_aligned(a->q, a->k_cache, a->v_cache))) {
-      if (stream_setup(p, a->dtype, a->cache_len) <= 0) return PF_ERR_LAUNCH;
-      return PF_OK;
-    }
-    if (stream_only(a->head_dim, a->dtype)) return PF_ERR_UNSUPPORTED;
+    if (*streams && stream_aligned(a->q, a->k_cache, a->v_cache))
+      return stream_setup(p, a->dtype, a->cache_len) > 0 ? PF_OK : PF_ERR_LAUNCH;
+    if (!*streams && only) return PF_ERR_UNSUPPORTED;
   }
-  p->chunk = decode_chunk(units, a->cache_len);
-  p->n_split = (a->cache_len + p->chunk - 1) / p->chunk;
-  if (units * p->n_split > kMaxGrid) return PF_ERR_UNSUPPORTED;
-  return PF_OK;
+  return generic_setup(p, a->cache_len, *streams && only ? stream_room(*p, a->dtype) : 0);
 }
 
 // The bytes of `slots` partials (max, sum and D accumulators each).
@@ -676,7 +695,7 @@ static size_t partial_bytes(size_t slots, int D) {
 // query rows -- at most one piece that a wave opens with and one that it ends
 // with --, generic kernel one per (b, query head, chunk).
 static size_t decode_slots(const pf::DecodeParams& p) {
-  if (p.n_waves == 0) return (size_t)p.B * p.Hq * p.n_split;
+  if (p.n_waves == 0) return (size_t)p.slice * p.Hq * p.n_split;
   const int group = p.Hq / p.Hkv;
   const int64_t seqs = (int64_t)p.B * p.Hkv * ((group + 15) / 16);
   return (size_t)(p.n_waves + (seqs < p.n_waves ? seqs : p.n_waves)) * pf::decode_stream_qrows(group);
@@ -686,15 +705,15 @@ static size_t decode_slots(const pf::DecodeParams& p) {
 // up to `cap` keys and wherever its operands lie, and for the streaming forms
 // whatever the batch -- a program asks once and keeps the workspace while its
 // sequences grow. So it counts two pieces for every wave of a full streaming
-// grid, and the generic kernel's chunks where a call can end up there.
+// grid, and the chunks that generic_setup makes without a bound.
 static size_t decode_ws_most(const pf::DecodeParams& p, int dtype, bool streams, int64_t cap) {
   const int group = p.Hq / p.Hkv;
   size_t most = 0;
+  if (streams && stream_only(p.dr, dtype)) return partial_bytes(stream_room(p, dtype), p.D);
   if (streams) {
     int waves = stream_grid(dtype, p.D, group, false);
     if (dtype == PF_DTYPE_F32 && p.D == 64) waves = std::max(waves, stream_grid(dtype, p.D, group, true));
     most = partial_bytes((size_t)2 * waves * pf::decode_stream_qrows(group), p.D);
-    if (stream_only(p.dr, dtype)) return most;
   }
   // decode_chunk's chunks have at least kMinChunk keys and at least cap / splits.
   const int64_t units = (int64_t)p.B * p.Hkv * ((group + 31) / 32);
@@ -706,20 +725,42 @@ static size_t decode_ws_most(const pf::DecodeParams& p, int dtype, bool streams,
 // The bytes that a launch insists on: what it uses; the 16-bit head_dim 128
 // forms the full size that their query answers (or more, where another thread
 // has just lowered decode_waves).
-static size_t decode_ws_bytes(const pf::DecodeParams& p, int dtype) {
+static size_t decode_ws_bytes(const pf::DecodeParams& p, int dtype, bool streams) {
   const size_t used = partial_bytes(decode_slots(p), p.D);
-  if (p.n_waves == 0 || !stream_only(p.dr, dtype)) return used;
+  if (!streams || !stream_only(p.dr, dtype)) return used;
   return std::max(used, decode_ws_most(p, dtype, true, 0));
 }
 
-static int bind_workspace(pf::DecodeParams* p, int dtype, void* ws, size_t bytes) {
-  const size_t need = decode_ws_bytes(*p, dtype);
+static int bind_workspace(pf::DecodeParams* p, int dtype, bool streams, void* ws, size_t bytes) {
+  const size_t need = decode_ws_bytes(*p, dtype, streams);
   if (need == 0) return PF_OK;
   if (!ws || bytes < need || ((uintptr_t)ws & 255) != 0) return PF_ERR_WORKSPACE;
   const size_t slots = decode_slots(*p);
   p->part_o = static_cast<float*>(ws);
   p->part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + align256(slots * p->D * sizeof(float)));
   return PF_OK;
+}
+
+// The launch: all of it, or the generic kernel slice after slice.
+static int run_decode(const pf::DecodeParams& p, int dtype, bool paged, hipStream_t stream) {
+  if (p.n_waves > 0 || p.slice >= p.B) return finish(pf::launch_decode(p, dtype, paged, stream));
+  const int64_t es = dtype == PF_DTYPE_F32 ? 4 : 2;
+  const int64_t q_bytes = (int64_t)p.Hq * p.dr * es, kv_bytes = paged ? 0 : (int64_t)p.Hkv * p.cache_size * p.dr * es;
+  int st = PF_OK;
+  for (int b = 0; b < p.B && st == PF_OK; b += p.slice) {
+    pf::DecodeParams s = p;
+    s.B = std::min(p.slice, p.B - b);
+    s.q = static_cast<const char*>(p.q) + b * q_bytes;
+    s.o = static_cast<char*>(p.o) + b * q_bytes;
+    s.k = static_cast<const char*>(p.k) + b * kv_bytes;
+    s.v = static_cast<const char*>(p.v) + b * kv_bytes;
+    if (paged) {
+      s.context_lens = p.context_lens + b;
+      if (p.block_tables != nullptr) s.block_tables = p.block_tables + (int64_t)b * p.pages_per_seq;
+    }
+    st = finish(pf::launch_decode(s, dtype, paged, stream));
+  }
+  return st;
 }
 
 size_t pf_attn_decode_workspace_size(const pf_attn_decode_args* a) {
@@ -736,9 +777,9 @@ int pf_attn_decode(const pf_attn_decode_args* a, void* stream) {
   if (st != PF_OK) return st;
   if (!a->q || !a->k_cache || !a->v_cache || !a->o) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, streams, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
-  return finish(pf::launch_decode(p, a->dtype, false, (hipStream_t)stream));
+  return run_decode(p, a->dtype, false, (hipStream_t)stream);
 }
 
 // most_ws: the partials' room, where it cannot grow (the streaming grid can be
@@ -756,7 +797,6 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p, bool* st
   const int64_t max_len = (int64_t)a->pages_per_seq * a->page_size;
   if (max_len > 0x7fffffff) return PF_ERR_UNSUPPORTED;
   const int g = a->num_heads / a->num_kv_heads;
-  const int64_t units = (int64_t)a->batch * a->num_kv_heads * ((g + 31) / 32);
   *p = pf::DecodeParams{};
   p->q = a->q;
   p->k = a->k_pages;
@@ -774,20 +814,16 @@ static int fill_paged(const pf_paged_attn_args* a, pf::DecodeParams* p, bool* st
   p->pages_per_seq = a->pages_per_seq;
   p->scale_log2 = a->sm_scale * 1.4426950408889634f;
   *streams = false;
+  const bool only = stream_only(a->head_dim, a->dtype);
   if (pf::decode_stream_supported(a->dtype, a->head_dim, g, true, a->page_size)) {
-    const bool only = stream_only(a->head_dim, a->dtype);
     *streams = stream_range_ok(a->page_size, a->head_dim, a->dtype);
-    if (*streams && (only || stream_aligned(a->q, a->k_pages, a->v_pages))) {
+    if (*streams && stream_aligned(a->q, a->k_pages, a->v_pages)) {
       if (stream_setup(p, a->dtype, max_len) <= 0) return PF_ERR_LAUNCH;
-      if (only || decode_ws_bytes(*p, a->dtype) <= most_ws) return PF_OK;
-      p->n_waves = 0;
+      if (only || decode_ws_bytes(*p, a->dtype, *streams) <= most_ws) return PF_OK;
     }
-    if (only) return PF_ERR_UNSUPPORTED;
+    if (!*streams && only) return PF_ERR_UNSUPPORTED;
   }
-  p->chunk = decode_chunk(units, (int)(max_len > 0 ? max_len : 1));
-  p->n_split = max_len > 0 ? (int)((max_len + p->chunk - 1) / p->chunk) : 1;
-  if (units * p->n_split > kMaxGrid) return PF_ERR_UNSUPPORTED;
-  return PF_OK;
+  return generic_setup(p, max_len > 0 ? max_len : 1, *streams && only ? stream_room(*p, a->dtype) : 0);
 }
 
 size_t pf_paged_attn_workspace_size(const pf_paged_attn_args* a) {
@@ -805,9 +841,9 @@ int pf_paged_attn(const pf_paged_attn_args* a, void* stream) {
   if (!a->q || !a->k_pages || !a->v_pages || !a->o || !a->context_lens) return PF_ERR_INVALID;
   if (a->pages_per_seq > 0 && !a->block_tables) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, streams, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
-  return finish(pf::launch_decode(p, a->dtype, true, (hipStream_t)stream));
+  return run_decode(p, a->dtype, true, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -864,13 +900,13 @@ int pf_paged_attn_noalloc(const pf_paged_attn_args* a, void* stream) {
   if (!a->q || !a->k_pages || !a->v_pages || !a->o || !a->context_lens) return PF_ERR_INVALID;
   if (a->pages_per_seq > 0 && !a->block_tables) return PF_ERR_INVALID;
   if (a->batch == 0) return PF_OK;
-  if (decode_ws_bytes(p, a->dtype) > (size_t)PF_NOALLOC_SCRATCH_BYTES) return PF_ERR_WORKSPACE;
+  if (decode_ws_bytes(p, a->dtype, streams) > (size_t)PF_NOALLOC_SCRATCH_BYTES) return PF_ERR_WORKSPACE;
   void* ws = nullptr;
   st = scratch_address((hipStream_t)stream, &ws);
   if (st != PF_OK) return st;
-  st = bind_workspace(&p, a->dtype, ws, PF_NOALLOC_SCRATCH_BYTES);
+  st = bind_workspace(&p, a->dtype, streams, ws, PF_NOALLOC_SCRATCH_BYTES);
   if (st != PF_OK) return st;
-  return finish(pf::launch_decode(p, a->dtype, true, (hipStream_t)stream));
+  return run_decode(p, a->dtype, true, (hipStream_t)stream);
 }
 
 int pf_rope(const pf_rope_args* a, void* stream) {
@@ -965,7 +1001,7 @@ static int fill_decode_step(const pf_attn_decode_step_args* a, pf::DecodeParams*
 size_t pf_attn_decode_step_workspace_size(const pf_attn_decode_step_args* a) {
   pf::DecodeParams p;
   if (fill_decode_step(a, &p) != PF_OK) return 0;
-  return decode_ws_bytes(p, a->dtype);
+  return decode_ws_bytes(p, a->dtype, true);
 }
 
 int pf_attn_decode_step(const pf_attn_decode_step_args* a, void* stream) {
@@ -975,8 +1011,9 @@ int pf_attn_decode_step(const pf_attn_decode_step_args* a, void* stream) {
   if (a->batch == 0) return PF_OK;
   if (!a->q || !a->k_new || !a->v_new || !a->k_cache || !a->v_cache || !a->o || !a->positions)
     return PF_ERR_INVALID;
-  st = bind_workspace(&p, a->dtype, a->workspace, a->workspace_bytes);
+  st = bind_workspace(&p, a->dtype, true, a->workspace, a->workspace_bytes);
   if (st != PF_OK) return st;
+  if (!stream_aligned(a->q, a->k_cache, a->v_cache)) return PF_ERR_INVALID;
   return finish(pf::launch_decode(p, a->dtype, false, (hipStream_t)stream));
 }
 

@@ -1,8 +1,8 @@
 // Single-query decode attention for gfx950: contiguous KV cache and paged pool,
 // in the forms the streaming kernel (decode_stream.hpp) does not take: head
 // dims between the kernel sizes (96, 200, ...), page sizes that are not a
-// multiple of 4 (8 for 128-byte rows), and, off 16-bit head_dim 128, groups of
-// more than 16 query heads.
+// multiple of 4 (8 for 128-byte rows), operands that lie between two 16-byte
+// boundaries, and, off 16-bit head_dim 128, groups of more than 16 query heads.
 //
 // Replaces `flash_attention_decode` (flash_attention.py:555-589: the forward
 // pallas_call with block_q = 1, kv_len = cache_len) and the

@@ -397,6 +397,8 @@ PyObject* paged(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
+bool aligned16(const Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
+
 // step(q, k_new, v_new, k_cache, v_cache, positions, cos, sin, ring, sm_scale)
 // -> o | None (the caches are written in place)
 PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -411,7 +413,8 @@ PyObject* step(PyObject*, PyObject* const* args, Py_ssize_t n) {
       kn->sizes() != vn->sizes() || kc->size(0) != q->size(0) || kn->size(0) != q->size(0) ||
       kn->size(1) != kc->size(1) || kn->size(2) != 1 || kn->size(3) != q->size(3) || !kc->is_contiguous() ||
       !vc->is_contiguous() || !ints_ok(pos, *q) || pos->dim() > 1 ||
-      (pos->numel() != 1 && pos->numel() != q->size(0)) || has_tangent({kn, vn}) || !get_bool(args[8], &ring) ||
+      (pos->numel() != 1 && pos->numel() != q->size(0)) || has_tangent({kn, vn}) || !aligned16(*kc) ||
+      !aligned16(*vc) || !aligned16(*q) || !get_bool(args[8], &ring) ||
       !get_scale(args[9], q->size(3), &scale))
     Py_RETURN_NONE;
   if (rot && (!cos || !sin || cos->dim() != 2 || !fits_i32(*cos) || !table_ok(cos, *q, cos->size(0)) ||

@@ -189,6 +189,14 @@ def flash_attention_decode_step(
     o = torch.empty_like(q)
     if batch == 0:
         return o
+    if any(t.data_ptr() % 16 for t in (q, k_cache, v_cache)):
+        # views between two 16-byte boundaries: through aligned copies
+        kc, vc = k_cache.detach().clone(), v_cache.detach().clone()
+        o = flash_attention_decode_step(q.detach().clone(), k_new, v_new, kc, vc, pos, cos, sin, ring=ring,
+                                        sm_scale=sm_scale)
+        k_cache.detach().copy_(kc)
+        v_cache.detach().copy_(vc)
+        return o
     args = _lib.DecodeStepArgs(
         _lib.ptr(q), _lib.ptr(k_new), _lib.ptr(v_new), _lib.ptr(k_cache), _lib.ptr(v_cache), _lib.ptr(o),
         _lib.ptr(pos), stride, _lib.ptr(cos), _lib.ptr(sin), 0 if cos is None else cos.shape[0],
