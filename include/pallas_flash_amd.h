@@ -99,7 +99,8 @@ int pf_attn_fwd(const pf_attn_fwd_args* args, void* stream);
  * `workspace`, which a second kernel merges; the results equal pf_attn_fwd's
  * to float32 rounding. pf_attn_fwd_workspace_size(args) bytes (0: this call
  * gains nothing from it, and workspace may be NULL), 256-byte aligned device
- * memory, contents on entry do not matter. A smaller one: PF_ERR_WORKSPACE. */
+ * memory, contents on entry do not matter; 200 MiB at most. A smaller one:
+ * PF_ERR_WORKSPACE. */
 size_t pf_attn_fwd_workspace_size(const pf_attn_fwd_args* args);
 int pf_attn_fwd_ws(const pf_attn_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 
@@ -205,7 +206,7 @@ int pf_attn_bwd_dkv(const pf_attn_bwd_args* args, void* stream);
 int pf_attn_bwd(const pf_attn_bwd_args* args, void* stream);
 /* pf_attn_bwd with a workspace (as pf_attn_fwd_ws): with few work items dQ runs
  * by chunks of keys and dK/dV by runs of query blocks, and a third kernel sums
- * their float32 partials. */
+ * their float32 partials; 400 MiB at most. */
 size_t pf_attn_bwd_workspace_size(const pf_attn_bwd_args* args);
 int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -123,6 +123,23 @@ def test_bwd_requires_buffers(L):
     assert L.pf_attn_bwd(a, None) == _lib.PF_ERR_INVALID
 
 
+@pytest.mark.parametrize("dtype,D", [(0, 64), (0, 128), (1, 64), (2, 128), (1, 256)])
+def test_split_workspace_is_bounded(L, dtype, D):
+    """Long few-headed calls, whose work items are few and whose rows are many:
+    the splits' partials stay within the stated size, and a split is still made."""
+    split = 0
+    for heads, kv in ((1, 1), (8, 1), (32, 1), (32, 8)):
+        for batch in (1, 2, 8):
+            for seq in (1024, 4096, 16384, 32768, 50000):
+                for causal in (0, 1):
+                    tail = (batch, heads, kv, seq, seq, D, seq, causal, 0.1, dtype)
+                    fwd = L.pf_attn_fwd_workspace_size(_lib.FwdArgs(*[8] * 5, *tail))
+                    bwd = L.pf_attn_bwd_workspace_size(_lib.BwdArgs(*[8] * 10, *tail))
+                    assert fwd <= 200 << 20 and bwd <= 400 << 20, tail
+                    split += bwd > 0
+    assert split > 20
+
+
 @pytest.mark.parametrize("sq,sk", [(1 << 22, 8), (8, 1 << 22), (1 << 23, 1 << 23)])
 def test_bwd_rejects_sequences_past_32bit_offsets(L, sq, sk):
     """The backward kernels address one head's rows with 32-bit byte offsets

@@ -200,10 +200,16 @@ constexpr double kStartUs = 5.0;        // a workgroup's prologue and epilogue
 constexpr double kSplitLaunchUs = 5.0;  // the second kernel
 constexpr double kPartialBytesPerUs = 4.0e6;
 constexpr int kMaxSplit = 64;
+// The partials of one kernel at most: a call must not need memory out of
+// proportion to its own. Without a bound the model alone asked up to 2 GiB (float32
+// dK/dV, 32/1 heads, 32768 keys, whose gradients are 544 MiB). At 192 MiB 1 in 100
+// causal training shapes of up to 8192 rows loses over 2% of its modelled time, the
+// worst 10%; at 128 MiB 2 in 100, the worst 37%; at 64 MiB 8 in 100, the worst 103%.
+constexpr int64_t kMaxPartialBytes = (int64_t)192 << 20;
 
 template <typename F>
 int plan_split(int64_t items, int max_steps, double total_steps, int min_per, double step_us, int64_t partial_bytes,
-               F grid) {
+               F grid) {  // partial_bytes: of one chunk of every item
   if (items <= 0 || items >= 2 * kCus) return 0;
   double best = kStartUs + step_us * fmax((double)max_steps, total_steps / kCus);
   int best_per = 0, last = 0;
@@ -212,6 +218,7 @@ int plan_split(int64_t items, int max_steps, double total_steps, int min_per, do
     per = (per + min_per - 1) / min_per * min_per;
     if (per >= max_steps || per == last) continue;
     last = per;
+    if ((max_steps + per - 1) / per * partial_bytes > kMaxPartialBytes) break;
     const double wgs = (double)grid(per);
     const double us = ceil(wgs / kCus) * (kStartUs + per * step_us) + kSplitLaunchUs +
                       2.0 * wgs / (double)items * (double)partial_bytes / kPartialBytesPerUs;
