@@ -230,6 +230,9 @@ int pf_attn_bwd_ws(const pf_attn_bwd_args* args, void* workspace, size_t workspa
  * depend on cache_len or on the pointers (which may be NULL in the query): ask
  * once for a cache and keep the workspace while it fills. For bf16/f16 with
  * head_dim 128 it is the same for every batch and cache_size, too.
+ * pf_attn_decode_workspace_min(args): what this one call insists on, with its
+ * cache_len and its pointers (at most the size above), for a caller that
+ * allocates per call.
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* q;
@@ -245,6 +248,7 @@ typedef struct {
 } pf_attn_decode_args;
 
 size_t pf_attn_decode_workspace_size(const pf_attn_decode_args* args);
+size_t pf_attn_decode_workspace_min(const pf_attn_decode_args* args);
 int pf_attn_decode(const pf_attn_decode_args* args, void* stream);
 
 /* ---------------------------------------------------------------------------
@@ -263,7 +267,7 @@ int pf_attn_decode(const pf_attn_decode_args* args, void* stream);
  * at head_dim 64), so that a load stays inside one page, the generic split-KV
  * kernel the others, with the same results to rounding.
  * workspace: at least pf_paged_attn_workspace_size(args) bytes; the size does
- * not depend on the context lengths or the pointers.
+ * not depend on the context lengths or the pointers (_min: as for the decode).
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* q;
@@ -281,6 +285,7 @@ typedef struct {
 } pf_paged_attn_args;
 
 size_t pf_paged_attn_workspace_size(const pf_paged_attn_args* args);
+size_t pf_paged_attn_workspace_min(const pf_paged_attn_args* args);
 int pf_paged_attn(const pf_paged_attn_args* args, void* stream);
 
 /* ---------------------------------------------------------------------------

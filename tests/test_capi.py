@@ -195,9 +195,15 @@ def test_decode_workspace_depends_on_the_shape_alone(L, dtype, D, heads, kv):
     sizes = {L.pf_attn_decode_workspace_size(_dec(cache_len=n, **p, **base))
              for n in (1, 63, 300, 1537, 4001, 6000, 8192) for p in (NULLS, ALIGNED, UNALIGNED)}
     assert len(sizes) == 1 and min(sizes) > 0
+    least = [L.pf_attn_decode_workspace_min(_dec(cache_len=n, **p, **base))
+             for n in (1, 63, 300, 1537, 4001, 6000, 8192) for p in (ALIGNED, UNALIGNED)]
+    assert 0 < min(least) and max(least) <= min(sizes)
     paged = {L.pf_paged_attn_workspace_size(_paged(k_pages=p["k_cache"], v_pages=p["v_cache"], q=p["q"], **base))
              for p in (NULLS, ALIGNED, UNALIGNED)}
     assert len(paged) == 1 and min(paged) > 0
+    for p in (ALIGNED, UNALIGNED):
+        assert 0 < L.pf_paged_attn_workspace_min(_paged(k_pages=p["k_cache"], v_pages=p["v_cache"], q=p["q"],
+                                                        **base)) <= min(paged)
     if D == 128 and dtype != 0:
         for other in (dict(batch=1), dict(batch=4096), dict(batch=1, cache_size=7, cache_len=7)):
             assert {L.pf_attn_decode_workspace_size(_dec(**{**base, **other}))} == sizes == paged

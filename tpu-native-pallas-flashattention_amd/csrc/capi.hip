@@ -777,6 +777,13 @@ size_t pf_attn_decode_workspace_size(const pf_attn_decode_args* a) {
   return decode_ws_most(p, a->dtype, streams, a->cache_size);
 }
 
+size_t pf_attn_decode_workspace_min(const pf_attn_decode_args* a) {
+  pf::DecodeParams p;
+  bool streams;
+  if (fill_decode(a, &p, &streams) != PF_OK) return 0;
+  return decode_ws_bytes(p, a->dtype, streams);
+}
+
 int pf_attn_decode(const pf_attn_decode_args* a, void* stream) {
   pf::DecodeParams p;
   bool streams;
@@ -838,6 +845,13 @@ size_t pf_paged_attn_workspace_size(const pf_paged_attn_args* a) {
   bool streams;
   if (fill_paged(a, &p, &streams, SIZE_MAX) != PF_OK) return 0;
   return decode_ws_most(p, a->dtype, streams, (int64_t)a->pages_per_seq * a->page_size);
+}
+
+size_t pf_paged_attn_workspace_min(const pf_paged_attn_args* a) {
+  pf::DecodeParams p;
+  bool streams;
+  if (fill_paged(a, &p, &streams, SIZE_MAX) != PF_OK) return 0;
+  return decode_ws_bytes(p, a->dtype, streams);
 }
 
 int pf_paged_attn(const pf_paged_attn_args* a, void* stream) {

@@ -356,7 +356,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     pf_attn_decode_args a{q1.data_ptr(), k1.data_ptr(), v1.data_ptr(), o.data_ptr(), (int32_t)q1.size(0),
                           (int32_t)q1.size(1), (int32_t)k1.size(1), (int32_t)k1.size(2), (int32_t)q1.size(3), len,
                           scale, dtype_tag(q1), nullptr, 0};
-    a.workspace_bytes = pf_attn_decode_workspace_size(&a);
+    a.workspace_bytes = pf_attn_decode_workspace_min(&a);
     if (a.workspace_bytes == 0) throw Declined();
     const Tensor ws = bytes(a.workspace_bytes, q1);
     a.workspace = ws.data_ptr();
@@ -388,7 +388,7 @@ PyObject* paged(PyObject*, PyObject* const* args, Py_ssize_t n) {
                          lens->data_ptr<int32_t>(), o.data_ptr(), (int32_t)q1.size(0), (int32_t)q1.size(1),
                          (int32_t)k->size(1), (int32_t)k->size(0), (int32_t)k->size(2), (int32_t)q1.size(3),
                          (int32_t)tab->size(1), scale, dtype_tag(q1), nullptr, 0};
-    a.workspace_bytes = pf_paged_attn_workspace_size(&a);
+    a.workspace_bytes = pf_paged_attn_workspace_min(&a);
     if (a.workspace_bytes == 0) throw Declined();
     const Tensor ws = bytes(a.workspace_bytes, q1);
     a.workspace = ws.data_ptr();

@@ -132,8 +132,10 @@ SIGNATURES = {
     "pf_attn_bwd_workspace_size": ([ctypes.POINTER(BwdArgs)], ctypes.c_size_t),
     "pf_attn_bwd_ws": ([ctypes.POINTER(BwdArgs), c_ptr, ctypes.c_size_t, c_ptr], ctypes.c_int),
     "pf_attn_decode_workspace_size": ([ctypes.POINTER(DecodeArgs)], ctypes.c_size_t),
+    "pf_attn_decode_workspace_min": ([ctypes.POINTER(DecodeArgs)], ctypes.c_size_t),
     "pf_attn_decode": ([ctypes.POINTER(DecodeArgs), c_ptr], ctypes.c_int),
     "pf_paged_attn_workspace_size": ([ctypes.POINTER(PagedArgs)], ctypes.c_size_t),
+    "pf_paged_attn_workspace_min": ([ctypes.POINTER(PagedArgs)], ctypes.c_size_t),
     "pf_paged_attn": ([ctypes.POINTER(PagedArgs), c_ptr], ctypes.c_int),
     "pf_paged_attn_noalloc": ([ctypes.POINTER(PagedArgs), c_ptr], ctypes.c_int),
     "pf_rope": ([ctypes.POINTER(RopeArgs), c_ptr], ctypes.c_int),

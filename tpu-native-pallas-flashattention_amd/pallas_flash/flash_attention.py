@@ -191,7 +191,7 @@ def _decode(q, k_cache, v_cache, cache_len: int, sm_scale: float):
         _lib.ptr(q), _lib.ptr(k_cache), _lib.ptr(v_cache), _lib.ptr(o),
         B, Hq, Hkv, cap, D, int(cache_len), float(sm_scale), _lib.dtype_tag(q), None, 0)
     L = _lib.lib()
-    ws_bytes = L.pf_attn_decode_workspace_size(args)
+    ws_bytes = L.pf_attn_decode_workspace_min(args)
     ws = torch.empty(max(int(ws_bytes), 1), dtype=torch.uint8, device=q.device)
     args.workspace = ws.data_ptr()
     args.workspace_bytes = ws.numel()

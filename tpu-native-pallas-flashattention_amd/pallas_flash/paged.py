@@ -101,7 +101,7 @@ def paged_flash_attention(
         _lib.ptr(o), batch, num_heads, num_kv_heads, num_pages, page_size, dp,
         tables.shape[1], float(sm_scale), _lib.dtype_tag(q), None, 0)
     L = _lib.lib()
-    ws_bytes = L.pf_paged_attn_workspace_size(args)
+    ws_bytes = L.pf_paged_attn_workspace_min(args)
     ws = torch.empty(max(int(ws_bytes), 1), dtype=torch.uint8, device=dev)
     args.workspace = ws.data_ptr()
     args.workspace_bytes = ws.numel()
