@@ -140,6 +140,32 @@ def test_split_workspace_is_bounded(L, dtype, D):
     assert split > 20
 
 
+def test_split_plans_take_the_same_time_at_any_length(L):
+    """The planner, which runs at every call, does not walk over the blocks of a
+    long sequence for every split it weighs: a call of tens of thousands of rows
+    plans within a few times a short one's time (both about 1 us; with such
+    loops 25 and 75 us)."""
+    import time
+
+    def us(fn, args):
+        best = float("inf")
+        for _ in range(20):
+            t = time.perf_counter()
+            for _ in range(20):
+                fn(args)
+            best = min(best, (time.perf_counter() - t) / 20 * 1e6)
+        return best
+
+    def both(seq):
+        tail = (1, 4, 1, seq, seq, 128, seq, 1, 0.1, 1)
+        return (us(L.pf_attn_fwd_workspace_size, _lib.FwdArgs(*[8] * 5, *tail)),
+                us(L.pf_attn_bwd_workspace_size, _lib.BwdArgs(*[8] * 10, *tail)))
+
+    short = both(1024)
+    for seq in (16000, 50000):
+        assert max(both(seq)) < 5 * max(short) + 5, seq
+
+
 @pytest.mark.parametrize("sq,sk", [(1 << 22, 8), (8, 1 << 22), (1 << 23, 1 << 23)])
 def test_bwd_rejects_sequences_past_32bit_offsets(L, sq, sk):
     """The backward kernels address one head's rows with 32-bit byte offsets

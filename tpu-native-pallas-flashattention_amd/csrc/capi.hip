@@ -184,7 +184,7 @@ pf::WorkTail plan_tail(int n_work, int min_items, hipStream_t stream) {
 // against the whole items' start + step x (the longest item's steps, or a CU's
 // share of all steps where that is more). Step times are measured, one
 // workgroup per CU (two resident ones take about twice as long per step, so
-// counting 256 at a time prices them alike). grid(per): the workgroups of that
+// counting 256 at a time prices them alike). wgs(per): the workgroups of that
 // chunk; min_per: the chunk's granularity.
 // ---------------------------------------------------------------------------
 struct StepCost {
@@ -209,7 +209,7 @@ constexpr int64_t kMaxPartialBytes = (int64_t)192 << 20;
 
 template <typename F>
 int plan_split(int64_t items, int max_steps, double total_steps, int min_per, double step_us, int64_t partial_bytes,
-               F grid) {  // partial_bytes: of one chunk of every item
+               F wgs) {  // partial_bytes: of one chunk of every item
   if (items <= 0 || items >= 2 * kCus) return 0;
   double best = kStartUs + step_us * fmax((double)max_steps, total_steps / kCus);
   int best_per = 0, last = 0;
@@ -219,9 +219,9 @@ int plan_split(int64_t items, int max_steps, double total_steps, int min_per, do
     if (per >= max_steps || per == last) continue;
     last = per;
     if ((max_steps + per - 1) / per * partial_bytes > kMaxPartialBytes) break;
-    const double wgs = (double)grid(per);
-    const double us = ceil(wgs / kCus) * (kStartUs + per * step_us) + kSplitLaunchUs +
-                      2.0 * wgs / (double)items * (double)partial_bytes / kPartialBytesPerUs;
+    const double n_wgs = wgs(per);
+    const double us = ceil(n_wgs / kCus) * (kStartUs + per * step_us) + kSplitLaunchUs +
+                      2.0 * n_wgs / (double)items * (double)partial_bytes / kPartialBytesPerUs;
     if (us < 0.95 * best) {
       best = us;
       best_per = per;
@@ -232,18 +232,20 @@ int plan_split(int64_t items, int max_steps, double total_steps, int min_per, do
 
 size_t align_ws(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Key blocks of 64 summed over query blocks of `rows` rows (one head, one
-// batch): all of kv_len, or up to the block's diagonal.
-double sum_key_blocks(int Sq, int rows, int kv_len, bool causal) {
-  const int nq = (Sq + rows - 1) / rows;
-  if (!causal) return (double)nq * ((kv_len + 63) / 64);
-  double t = 0;
-  for (int i = 0; i < nq; ++i) {
-    const int64_t end = (int64_t)(i + 1) * rows;
-    const int e = (int)(end < Sq ? end : Sq);
-    t += ((e < kv_len ? e : kv_len) + 63) / 64;
-  }
-  return t;
+// Workgroups of the key split into chunks of 64 per keys, for one head of one
+// batch: chunks summed over the query blocks of `rows` (32, 64 or 128) rows, which
+// need all of kv_len, or up to their diagonal. (per = 1: the steps.) Chunk c is
+// needed by all blocks but the first floor(64 per c / rows). In closed form: the
+// planner asks for some 20 values of per, where a loop over the blocks took 23 us
+// at 16000 rows.
+double key_split_grid(int Sq, int rows, int kv_len, int per, bool causal) {
+  const double nq = (Sq + rows - 1) / rows;
+  const int keys = causal && Sq < kv_len ? Sq : kv_len;
+  const int n = (int)((keys + (int64_t)64 * per - 1) / ((int64_t)64 * per));
+  if (!causal) return nq * n;
+  const double sum_c = 0.5 * n * (n - 1.0);
+  const double skipped = rows == 128 ? 0.5 * (per * sum_c - (per % 2 != 0 ? n / 2 : 0)) : 64 / rows * (per * sum_c);
+  return nq * n - skipped;
 }
 
 int chunks_of(int q0, int rows, int Sq, int kv_len, int chunk, bool causal) {
@@ -260,18 +262,16 @@ size_t plan_fwd_split(const pf_attn_fwd_args* a, pf::FwdParams* p) {
   const int max_steps = (max_keys + 63) / 64;
   if (max_steps <= 1) return 0;
   const int64_t rows = (int64_t)a->batch * a->num_heads * a->seq_len_q;
-  const double total = sum_key_blocks(a->seq_len_q, p->rpw, a->kv_len, a->causal != 0) * (p->n_work / p->n_qblk);
+  const int members = p->n_work / p->n_qblk;
+  const auto wgs = [&](int per) { return members * key_split_grid(a->seq_len_q, p->rpw, a->kv_len, per, a->causal); };
   const int min_per = a->causal && p->rpw > 64 ? 2 : 1;  // whole multiples of rpw
-  const auto grid = [&](int per) {
-    int64_t n = 0;
-    for (int i = 0; i < p->n_qblk; ++i) n += chunks_of(i * p->rpw, p->rpw, a->seq_len_q, a->kv_len, 64 * per, a->causal);
-    return n * (p->n_work / p->n_qblk);
-  };
-  const int per = plan_split(p->n_work, max_steps, total, min_per, step_cost(a->dtype, a->head_dim).fwd,
-                             rows * a->head_dim * 4, grid);
+  const int per = plan_split(p->n_work, max_steps, wgs(1), min_per, step_cost(a->dtype, a->head_dim).fwd,
+                             rows * a->head_dim * 4, wgs);
   if (per == 0) return 0;
   p->chunk = per * 64;
-  p->split_grid = (int)grid(per);
+  p->split_grid = 0;
+  for (int i = 0; i < p->n_qblk; ++i)
+    p->split_grid += chunks_of(i * p->rpw, p->rpw, a->seq_len_q, a->kv_len, p->chunk, a->causal) * members;
   p->n_split = (max_steps + per - 1) / per;
   const size_t prow = (size_t)p->n_split * rows;
   return align_ws(prow * a->head_dim * 4) + align_ws(prow * 8);
@@ -462,16 +462,13 @@ static size_t plan_bwd_split(const pf_attn_bwd_args* a, pf::BwdParams* p, size_t
   const int kb = (max_keys + 63) / 64;
   const int64_t dq_items = (int64_t)p->B * p->Hq * ((p->Sq + 127) / 128);
   if (kb > 1 && dq_items < 2 * kCus) {
-    const double total = sum_key_blocks(p->Sq, 128, p->kv_len, causal) * p->B * p->Hq;
-    const auto grid = [&](int per) {
-      int64_t n = 0;
-      for (int q0 = 0; q0 < p->Sq; q0 += 128) n += chunks_of(q0, 128, p->Sq, p->kv_len, 64 * per, causal);
-      return n * p->B * p->Hq;
-    };
-    const int per = plan_split(dq_items, kb, total, 1, cost.dq, rows_q * a->head_dim * 4, grid);
+    const auto wgs = [&](int per) { return (double)p->B * p->Hq * key_split_grid(p->Sq, 128, p->kv_len, per, causal); };
+    const int per = plan_split(dq_items, kb, wgs(1), 1, cost.dq, rows_q * a->head_dim * 4, wgs);
     if (per > 0) {
       p->chunk_q = per * 64;
-      p->grid_q = (int)grid(per);
+      p->grid_q = 0;
+      for (int q0 = 0; q0 < p->Sq; q0 += 128)
+        p->grid_q += chunks_of(q0, 128, p->Sq, p->kv_len, p->chunk_q, causal) * p->B * p->Hq;
       p->n_split_q = (kb + per - 1) / per;
       *dq_bytes = align_ws((size_t)p->n_split_q * rows_q * a->head_dim * 4);
     }
@@ -482,19 +479,24 @@ static size_t plan_bwd_split(const pf_attn_bwd_args* a, pf::BwdParams* p, size_t
   if (items * halves < 2 * kCus) {
     const int64_t max_steps = (int64_t)((p->Sq + bmq - 1) / bmq) * p->g;
     if (max_steps <= 0x7fffffff) {
-      double total = 0;
-      for (int64_t i = 0; i < nk; ++i) total += pf::dkv_steps(*p, (int)(128 * i), bmq, causal);
-      const auto grid = [&](int per) {
-        int64_t n = 0;
-        p->steps_k = per;
-        for (int64_t i = 0; i < nk; ++i) n += pf::dkv_runs(*p, (int)(128 * i), bmq, causal);
-        return n * p->B * p->Hkv * halves;
+      // As key_split_grid, over key blocks: block i < busy has (nqb - r i) g steps
+      // (not causal: nqb g), the others none, and every block at least one run.
+      const int64_t nqb = (p->Sq + bmq - 1) / bmq, r = 128 / bmq, members = (int64_t)p->B * p->Hkv * halves;
+      const int64_t busy = ((causal && p->Sq < p->kv_len ? p->Sq : p->kv_len) + 127) / 128;
+      const double total = (double)p->g * (busy * nqb - (causal ? r * (busy * (busy - 1) / 2) : 0));
+      const auto wgs = [&](int per) {
+        int64_t n = nk - busy;
+        if (!causal) n += busy * ((max_steps + per - 1) / per);
+        for (int64_t c = 0; causal && c < max_steps; c += per)  // run c / per: the blocks with more than c steps
+          n += std::min(busy, (nqb - 1 - c / p->g) / r + 1);
+        return (double)(n * members);
       };
-      const int per = plan_split(items * halves, (int)max_steps, total * p->B * p->Hkv * halves, 1, cost.dkv,
-                                 2 * rows_k * a->head_dim * 4, grid);
+      const int per = plan_split(items * halves, (int)max_steps, total * members, 1, cost.dkv,
+                                 2 * rows_k * a->head_dim * 4, wgs);
       p->steps_k = per;
       if (per > 0) {
-        p->grid_k = (int)(grid(per) / halves);
+        p->grid_k = 0;
+        for (int64_t i = 0; i < nk; ++i) p->grid_k += pf::dkv_runs(*p, (int)(128 * i), bmq, causal) * p->B * p->Hkv;
         p->n_split_k = (int)((max_steps + per - 1) / per);
         *dkv_bytes = align_ws((size_t)p->n_split_k * rows_k * a->head_dim * 4);
       }
