@@ -22,10 +22,12 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include <array>
 #include <climits>
 #include <cmath>
+#include <cstring>
 #include <exception>
 #include <initializer_list>
 
@@ -446,4 +448,17 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_calls", nullptr, -1, method
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_calls() { return PyModule_Create(&module); }
+// Built against one torch release's C++ interfaces: refuses to be imported under
+// another one, whose layouts may differ even where every symbol is found.
+PyMODINIT_FUNC PyInit__torch_calls() {
+  PyObject* torch = PyImport_ImportModule("torch");
+  if (torch == nullptr) return nullptr;
+  PyObject* version = PyObject_GetAttrString(torch, "__version__");
+  Py_DECREF(torch);
+  const char* v = version != nullptr ? PyUnicode_AsUTF8(version) : nullptr;
+  const size_t n = sizeof(TORCH_VERSION) - 1;
+  const bool same = v != nullptr && std::strncmp(v, TORCH_VERSION, n) == 0 && (v[n] == 0 || v[n] == '+');
+  if (!same && !PyErr_Occurred()) PyErr_Format(PyExc_ImportError, "built for torch %s, not %s", TORCH_VERSION, v);
+  Py_XDECREF(version);
+  return same ? PyModule_Create(&module) : nullptr;
+}

@@ -9,6 +9,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import warnings
 from typing import Iterator, Optional
 
 import torch
@@ -171,23 +172,32 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+class _Declining:
+    """Stands in for _torch_calls: declines every call."""
+
+    attention = rope = decode = paged = step = staticmethod(lambda *args: None)
+
+
 _calls = None
 
 
 def calls():
     """The C++ host side of the public calls (csrc/torch_calls.cpp). Each of
     its functions returns None for anything but the plain case, and the caller
-    then runs its general path."""
+    then runs its general path. Where the extension is not built, or built for
+    another Python or torch, every call runs that path: the same kernels and
+    results, some 20 to 100 us of Python later."""
     global _calls
     if _calls is None:
-        lib()
         try:
-            from . import _torch_calls
+            from . import _torch_calls as found
         except ImportError as e:
-            raise RuntimeError(
-                "_torch_calls.so is not built (or not for this torch); run `make` in "
-                "tpu-native-pallas-flashattention_amd/ or __graft_entry__.build()") from e
-        _calls = _torch_calls
+            found = _Declining
+            if os.path.exists(library_path()):  # without it lib() says what is missing
+                warnings.warn(f"the C++ host side of the public calls cannot be imported ({e}); calls go through "
+                              "Python. Run `make` in tpu-native-pallas-flashattention_amd/ or __graft_entry__.build()",
+                              RuntimeWarning, stacklevel=3)
+        _calls = found
     return _calls
 
 
