@@ -15,13 +15,15 @@
 
 from __future__ import annotations
 
+import contextlib
+
 import numpy as np
 import pytest
 import torch
 
 from gpu_util import DEV, TORCH_DT, check_fwd, dev, host, max_abs, note
 from oracle import cache_write_ref, decode_step_ref, paged_ref, paged_write_ref, precompute_rope_ref
-from pallas_flash import (flash_attention_decode_step, paged_flash_attention, precompute_rope,
+from pallas_flash import (_lib, flash_attention_decode_step, paged_flash_attention, precompute_rope,
                           write_kv_cache, write_to_paged_cache)
 
 pytestmark = pytest.mark.gpu
@@ -167,6 +169,13 @@ def test_cache_writes_out_of_place(which):
 
 
 # -------------------------------------------------------------- decode step --
+# Short caches run a workgroup per sequence by default (at most 384 slots); a
+# hand-set grid of w waves and longer caches run the persistent grid: 1 wave
+# walks every sequence, 7 cut them and cross from one to the next mid-range.
+def _waves(w):
+    return contextlib.nullcontext() if w is None else _lib.tuning(decode_waves=w)
+
+
 def _step_inputs(rng, B, Hq, Hkv, C, D, dt):
     return (dev(rng.standard_normal((B, Hq, 1, D)), dt), dev(rng.standard_normal((B, Hkv, 1, D)), dt),
             dev(rng.standard_normal((B, Hkv, 1, D)), dt), dev(rng.standard_normal((B, Hkv, C, D)), dt),
@@ -197,21 +206,23 @@ def _check_step(dt, q, kn, vn, kc0, vc0, kc, vc, o, pos, cos, sin, ring):
             assert max_abs(host(kc)[b][:, slot], kc_ref[b][:, slot]) <= 2e-2
 
 
-@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("dt,C,w", [("bf16", 200, None), ("f16", 200, None), ("bf16", 200, 1), ("f16", 200, 7),
+                                    ("bf16", 420, None)])
 @pytest.mark.parametrize("Hq,Hkv", [(8, 2), (32, 8), (4, 4), (32, 1), (24, 1)])
 @pytest.mark.parametrize("ring", [False, True])
-def test_decode_step_matches_oracle(dt, Hq, Hkv, ring):
+def test_decode_step_matches_oracle(dt, C, w, Hq, Hkv, ring):
     """(32, 1) and (24, 1): the group spans two 16-head slices, each of which
     streams (and patches) the new token's stage; only slice 0 writes the cache."""
-    note(f"decode_step dt={dt} Hq={Hq} Hkv={Hkv} ring={ring}")
+    note(f"decode_step dt={dt} C={C} waves={w} Hq={Hq} Hkv={Hkv} ring={ring}")
     rng = np.random.default_rng(15)
-    B, C, D = 4, 200, 128
+    B, D = 4, 128
     q, kn, vn, kc, vc = _step_inputs(rng, B, Hq, Hkv, C, D, dt)
     kc0, vc0 = kc.clone(), vc.clone()
     cos, sin = precompute_rope(1024, D, 10000.0, device=DEV)
-    pos = [0, 77, 199, 531] if ring else [0, 77, 199, 31]
-    o = flash_attention_decode_step(q, kn, vn, kc, vc, torch.tensor(pos, dtype=torch.int32, device=DEV),
-                                    cos, sin, ring=ring)
+    pos = [0, 77, C - 1, 531] if ring else [0, 77, C - 1, 31]
+    with _waves(w):
+        o = flash_attention_decode_step(q, kn, vn, kc, vc, torch.tensor(pos, dtype=torch.int32, device=DEV),
+                                        cos, sin, ring=ring)
     torch.cuda.synchronize()
     _check_step(dt, q, kn, vn, kc0, vc0, kc, vc, o, pos, cos, sin, ring)
 
@@ -225,40 +236,45 @@ def test_decode_step_without_rope_and_scalar_position():
     _check_step("bf16", q, kn, vn, kc0, vc0, kc, vc, o, 40, None, None, False)
 
 
-def test_decode_step_invalid_positions_write_nothing():
+@pytest.mark.parametrize("C,w", [(64, None), (64, 1), (64, 7), (420, None)])
+def test_decode_step_invalid_positions_write_nothing(C, w):
+    note(f"decode_step invalid positions C={C} waves={w}")
     rng = np.random.default_rng(17)
-    q, kn, vn, kc, vc = _step_inputs(rng, 4, 8, 2, 64, 128, "bf16")
+    q, kn, vn, kc, vc = _step_inputs(rng, 4, 8, 2, C, 128, "bf16")
     kc0, vc0 = kc.clone(), vc.clone()
-    cos, sin = precompute_rope(100, 128, 10000.0, device=DEV)
-    pos = [-3, 64, 10, 100]  # negative, past the capacity, valid, past the RoPE table
-    o = flash_attention_decode_step(q, kn, vn, kc, vc, torch.tensor(pos, dtype=torch.int32, device=DEV),
-                                    cos, sin)
+    cos, sin = precompute_rope(C + 36, 128, 10000.0, device=DEV)
+    pos = [-3, C, 10, C + 36]  # negative, past the capacity, valid, past the RoPE table
+    with _waves(w):
+        o = flash_attention_decode_step(q, kn, vn, kc, vc, torch.tensor(pos, dtype=torch.int32, device=DEV),
+                                        cos, sin)
     torch.cuda.synchronize()
     oh = host(o)
     assert not oh[[0, 1, 3]].any()
     _check_step("bf16", q, kn, vn, kc0, vc0, kc, vc, o, pos, cos, sin, False)
 
 
-def test_decode_step_ring_loop_matches_oracle():
+@pytest.mark.parametrize("C,first,w", [(40, 0, None), (40, 0, 1), (40, 0, 7), (420, 380, None)])
+def test_decode_step_ring_loop_matches_oracle(C, first, w):
     """A generate_streaming-style loop (model.py:406-531) on the attention
-    path: every step writes one token into a ring of 40 slots and attends the
-    live window; sequences start at different positions and wrap."""
-    note("decode_step ring loop")
+    path: every step writes one token into a ring of C slots and attends the
+    live window; the sequences wrap."""
+    note(f"decode_step ring loop C={C} waves={w}")
     rng = np.random.default_rng(18)
-    B, Hq, Hkv, C, D, T = 3, 8, 2, 40, 128, 90
+    B, Hq, Hkv, D, T = 3, 8, 2, 128, 90
     cos, sin = precompute_rope(512, D, 10000.0, device=DEV)
     kc = dev(np.zeros((B, Hkv, C, D)), "bf16")
     vc = dev(np.zeros((B, Hkv, C, D)), "bf16")
     kc_ref = np.zeros((B, Hkv, C, D))
     vc_ref = np.zeros((B, Hkv, C, D))
-    start = np.array([0, 0, 0], np.int64)
+    start = np.full(3, first, np.int64)
     pos = torch.tensor(start, dtype=torch.int32, device=DEV)
     worst = 0.0
     for t in range(T):
         q = dev(rng.standard_normal((B, Hq, 1, D)), "bf16")
         kn = dev(rng.standard_normal((B, Hkv, 1, D)), "bf16")
         vn = dev(rng.standard_normal((B, Hkv, 1, D)), "bf16")
-        o = flash_attention_decode_step(q, kn, vn, kc, vc, pos, cos, sin, ring=True)
+        with _waves(w):
+            o = flash_attention_decode_step(q, kn, vn, kc, vc, pos, cos, sin, ring=True)
         o_ref, kc_ref, vc_ref = decode_step_ref(host(q), host(kn), host(vn), kc_ref, vc_ref, start + t,
                                                 host(cos), host(sin), ring=True, store=_rounder("bf16"))
         worst = max(worst, max_abs(host(o), o_ref))
@@ -268,35 +284,37 @@ def test_decode_step_ring_loop_matches_oracle():
     assert max_abs(host(kc), kc_ref) <= 2e-2 and np.array_equal(host(vc), vc_ref)
 
 
-def test_decode_step_graph_replay_advances_positions_on_device():
+@pytest.mark.parametrize("C,w", [(64, None), (64, 7), (420, None)])
+def test_decode_step_graph_replay_advances_positions_on_device(C, w):
     """One captured decode step replayed while the positions advance on the
     GPU (no host-side value depends on them): every replay equals the eager
     step at that position."""
-    note("decode_step graph replay")
+    note(f"decode_step graph replay C={C} waves={w}")
     rng = np.random.default_rng(19)
-    B, Hq, Hkv, C, D = 2, 8, 2, 64, 128
-    cos, sin = precompute_rope(256, D, 10000.0, device=DEV)
+    B, Hq, Hkv, D = 2, 8, 2, 128
+    cos, sin = precompute_rope(C + 192, D, 10000.0, device=DEV)
     q, kn, vn, kc, vc = _step_inputs(rng, B, Hq, Hkv, C, D, "bf16")
     kc_e, vc_e = kc.clone(), vc.clone()
-    pos = torch.tensor([5, 30], dtype=torch.int32, device=DEV)
+    pos = torch.tensor([C - 59, C - 34], dtype=torch.int32, device=DEV)
     pos_e = pos.clone()
     # warm up on a side stream (allocator), then capture
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(s):
-        flash_attention_decode_step(q, kn, vn, kc.clone(), vc.clone(), pos.clone(), cos, sin, ring=True)
-    torch.cuda.current_stream().wait_stream(s)
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        o_g = flash_attention_decode_step(q, kn, vn, kc, vc, pos, cos, sin, ring=True)
-    for step in range(70):  # wraps the 64-slot ring
-        graph.replay()
-        o_e = flash_attention_decode_step(q, kn, vn, kc_e, vc_e, pos_e, cos, sin, ring=True)
+    with _waves(w):
+        with torch.cuda.stream(s):
+            flash_attention_decode_step(q, kn, vn, kc.clone(), vc.clone(), pos.clone(), cos, sin, ring=True)
+        torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
-        assert torch.equal(o_g, o_e), f"replay {step}"
-        pos += 1
-        pos_e += 1
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            o_g = flash_attention_decode_step(q, kn, vn, kc, vc, pos, cos, sin, ring=True)
+        for step in range(70):  # wraps the ring
+            graph.replay()
+            o_e = flash_attention_decode_step(q, kn, vn, kc_e, vc_e, pos_e, cos, sin, ring=True)
+            torch.cuda.synchronize()
+            assert torch.equal(o_g, o_e), f"replay {step}"
+            pos += 1
+            pos_e += 1
     assert torch.equal(kc, kc_e) and torch.equal(vc, vc_e)
 
 
