@@ -15,7 +15,9 @@ import types
 
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils.checkpoint import checkpoint
 
 from gpu_util import note
 from pallas_flash import (_lib, flash_attention, flash_attention_decode, flash_attention_decode_step,
@@ -31,6 +33,25 @@ def _declining():
     """The general path alone."""
     real = _lib.calls()
     _lib._calls = types.SimpleNamespace(**{n: (lambda *a: None) for n in NAMES})
+    try:
+        yield
+    finally:
+        _lib._calls = real
+
+
+@contextlib.contextmanager
+def _recording(seen):
+    """The C++ host side; notes which function was offered a call and whether it took it."""
+    real = _lib.calls()
+
+    def noting(name):
+        def call(*args):
+            o = getattr(real, name)(*args)
+            seen.append((name, o is not None))
+            return o
+        return call
+
+    _lib._calls = types.SimpleNamespace(**{n: noting(n) for n in NAMES})
     try:
         yield
     finally:
@@ -61,7 +82,7 @@ def _calls(dt):
         return (o, *torch.autograd.grad(o.sum(), ts))
 
     def step():
-        qs, ks, vs = _qkv(torch.bfloat16, S=64, D=128)
+        qs, ks, vs = _qkv(dt, S=64, D=128)
         c, s = (t.cuda() for t in precompute_rope(200, 128, 10000.0))
         pos = torch.tensor([3, 190], dtype=torch.int32, device="cuda")
         o = flash_attention_decode_step(qs[:, :, :1], ks[:, :, 5:6], vs[:, :, 7:8], ks, vs, pos, c, s, ring=True)
@@ -80,13 +101,20 @@ def _calls(dt):
     }
 
 
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("name", ["forward", "transposed", "train", "rope", "rope own tables", "decode", "paged",
-                                  "step"])
+DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+TAKEN_BY = {"forward": "attention", "transposed": "attention", "train": "attention", "rope": "rope",
+            "rope own tables": "rope", "decode": "decode", "paged": "paged", "step": "step"}
+
+
+@pytest.mark.parametrize("name,dt", [(n, dt) for n in TAKEN_BY for dt in DTYPES
+                                     if n != "step" or dt != torch.float32])  # the step is 16-bit
 def test_same_as_the_general_path(name, dt):
     note(f"calls: {name} {dt}")
     call = _calls(dt)[name]
-    got = call()
+    seen = []
+    with _recording(seen):
+        got = call()
+    assert seen == [(TAKEN_BY[name], True)]
     with _declining():
         want = call()
     assert len(got) == len(want)
@@ -143,6 +171,50 @@ def test_declines_what_it_does_not_know():
     with torch.autograd.forward_ad.dual_level():
         seen.append(c.attention(torch.autograd.forward_ad.make_dual(q, q), k, v, True, None, None))
     assert seen == [None, None, None]
+
+
+def test_tracer_and_function_mode_reach_the_general_path():
+    note("calls: jit tracer, function mode")
+    c = _lib.calls()
+    q, k, v = _qkv(torch.bfloat16)
+    want = flash_attention(q, k, v, causal=True)
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        seen.append(c.attention(q, k, v, True, None, None))
+        assert torch.equal(flash_attention(q, k, v, causal=True), want)
+    torch.jit.trace(lambda x: seen.append(c.attention(x, k, v, True, None, None)) or x * 1, (q,), check_trace=False)
+    assert seen == [None, None]
+    assert c.attention(q, k, v, True, None, None) is not None  # and afterwards it is taken again
+
+
+def test_create_graph_and_checkpoint():
+    """create_graph: the gradients are as the general path's, which are not
+    differentiable again. Checkpointing: the recomputation ends with an exception
+    that its pack hook throws through the C++ function."""
+    note("calls: create_graph, checkpoint")
+    ts = [t.requires_grad_(True) for t in _qkv(torch.float32)]
+    call = lambda *a: flash_attention(*a, causal=True)
+
+    def create_graph():
+        o = call(*ts)
+        return (o, *torch.autograd.grad(o.sum(), ts, create_graph=True))
+
+    got = create_graph()
+    with _declining():
+        want = create_graph()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b) and a.requires_grad == b.requires_grad
+    assert not got[1].requires_grad
+    seen = []
+    with _recording(seen):
+        grads = torch.autograd.grad(checkpoint(call, *ts, use_reentrant=False).sum(), ts)
+    assert ("attention", True) in seen
+    assert all(torch.equal(a, b) for a, b in zip(grads, want[1:]))
 
 
 def test_saved_tensor_hooks_and_graph_reuse():
