@@ -178,7 +178,7 @@ def test_bwd_rejects_sequences_past_32bit_offsets(L, sq, sk):
 
 
 def _dec(**over):
-    base = dict(q=8, k_cache=8, v_cache=8, o=8, batch=64, num_heads=32, num_kv_heads=8,
+    base = dict(q=256, k_cache=512, v_cache=1024, o=2048, batch=64, num_heads=32, num_kv_heads=8,
                 cache_size=8192, head_dim=128, cache_len=6000, sm_scale=0.1, dtype=1,
                 workspace=None, workspace_bytes=0)
     base.update(over)
@@ -236,7 +236,7 @@ def test_decode_workspace_depends_on_the_shape_alone(L, dtype, D, heads, kv):
 
 
 def _paged(**over):
-    base = dict(q=8, k_pages=8, v_pages=8, block_tables=8, context_lens=8, o=8, batch=128,
+    base = dict(q=256, k_pages=512, v_pages=1024, block_tables=8, context_lens=8, o=2048, batch=128,
                 num_heads=32, num_kv_heads=8, num_pages=16384, page_size=64, head_dim=128,
                 pages_per_seq=128, sm_scale=0.1, dtype=1, workspace=None, workspace_bytes=0)
     base.update(over)
@@ -333,7 +333,7 @@ def test_paged_cache_write_rejects_on_host(L, over, status):
 
 
 def _step(**over):
-    base = dict(q=8, k_new=8, v_new=8, k_cache=8, v_cache=8, o=8, positions=8, positions_stride=1,
+    base = dict(q=256, k_new=8, v_new=8, k_cache=512, v_cache=1024, o=2048, positions=8, positions_stride=1,
                 cos=8, sin=8, rope_len=8192, batch=64, num_heads=32, num_kv_heads=8, cache_size=8192,
                 head_dim=128, ring=0, sm_scale=0.1, dtype=1, workspace=None, workspace_bytes=0)
     base.update(over)

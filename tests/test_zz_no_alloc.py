@@ -6,8 +6,8 @@ with a caller workspace, on two calls in a row where the second is smaller
 (the array keeps the first call's contents), on the streaming kernel
 (bf16, page 64 and page 16), on a small persistent grid that cuts sequences
 across waves (partials in the array), at head_dim 256, and on the generic
-kernel (float32, page size 5); sizes past the array are refused before
-any launch.
+kernel (page size 5, float32 and head_dim 256); sizes past the array are
+refused before any launch.
 A call recorded into a HIP graph replays correctly while its inputs change
 in place, also when it is the process's first call of the entry point (the
 array's address is then looked up during the recording).
@@ -75,6 +75,7 @@ CASES = [  # (name, dt, page, Hq, Hkv, decode_waves, head_dim)
     ("stream bf16 page 16, 7-wave grid", "bf16", 16, 16, 2, 7, 128),
     ("generic f32 page 5", "f32", 5, 8, 2, 0, 128),
     ("stream bf16 head_dim 256 page 16", "bf16", 16, 8, 2, 0, 256),
+    ("generic bf16 head_dim 256 page 5", "bf16", 5, 8, 2, 0, 256),
 ]
 
 
