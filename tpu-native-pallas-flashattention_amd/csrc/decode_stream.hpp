@@ -44,7 +44,8 @@
 //  * A sequence whose stages all fall in one wave is finished by that wave
 //    (o = acc / l, l == 0 -> 0; flash_attention.py:150-159, paged.py:95-99).
 //    A sequence cut by wave boundaries leaves one partial (max, sum, acc)
-//    per piece (slot piece_slot); pf_decode_stream_combine_kernel merges them.
+//    per piece (slot piece_slot); pf_decode_stream_cut_kernel or
+//    pf_decode_stream_combine_kernel merges them (launch_combine).
 //
 // LDS stage layout: row-major SK x RB-byte tiles with the 16-byte chunks of
 // row r permuted by chunk ^ swz(r) (StreamGeo). Both read patterns are
@@ -265,124 +266,144 @@ __device__ inline void cursor_next(Cursor& c, const DecodeParams& p, int J) {
   c.nst = (c.L + SK - 1) / SK;
 }
 
-// Stage totals: per batch b, T_b = ceil(L_b / SK) * J stages. With s < 0
-// returns the total S; otherwise also fills *out with the cursor of global
-// stage s (which must be < S).
-template <int PG, int SK>
-__device__ inline int64_t locate(const DecodeParams& p, int J, int64_t s, Cursor* out) {
+__device__ inline int64_t readlane64(int64_t x, int lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)x >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+// Inclusive scan over the 64 lanes.
+__device__ inline int64_t scan64(int64_t x) {
   const int lane = threadIdx.x & 63;
-  if constexpr (PG == 0) {
-    const int nst = (p.cache_len + SK - 1) / SK;
-    const int64_t per_b = (int64_t)nst * J;
-    if (s >= 0) {
-      int64_t r, st;
-      int b;
-      if (p.B == 1) {
-        b = 0;
-        r = s;
-      } else if ((per_b >> 31) == 0) {
-        b = (int)div_pos(s, (int)per_b, &r);
-      } else {
-        b = (int)(s / per_b);
-        r = s % per_b;
-      }
-      const int j = (int)div_pos(r, nst, &st);
-      *out = Cursor{uni(b), uni(j), uni((int)st), uni(nst), uni(p.cache_len)};
-    }
-    return uni64(per_b * p.B);
-  } else {
-    int64_t base = 0;
-    for (int b0 = 0; b0 < p.B; b0 += 64) {
-      const int bb = b0 + lane;
-      const int Lb = bb < p.B ? len_lane<PG>(p, bb) : 0;
-      const int64_t t = (int64_t)((Lb + SK - 1) / SK) * J;
-      int64_t incl = t;  // inclusive scan over the 64 lanes
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int64_t y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-      }
-      const int64_t tot = __shfl(incl, 63);
-      if (s >= base && s < base + tot) {
-        const uint64_t hit = __ballot(base + incl > s);
-        const int ln = __builtin_ctzll(hit);
-        const int64_t excl = __shfl(incl - t, ln);
-        const int Lh = __shfl(Lb, ln);
-        const int nst = (Lh + SK - 1) / SK;
-        int64_t st;
-        const int j = (int)div_pos(s - base - excl, nst, &st);
-        *out = Cursor{uni(b0 + ln), uni(j), uni((int)st), uni(nst), uni(Lh)};
-        return -1;  // found (the total is not needed after the search)
-      }
-      base += tot;
-    }
-    return uni64(base);
+  for (int o = 1; o < 64; o <<= 1) {
+    const int64_t y = __shfl_up(x, o);
+    if (lane >= o) x += y;
   }
+  return x;
 }
 
-// With at most 64 batches one load of the per-batch lengths (a lane per
-// batch) gives everything both kernels need: lane bb's stage count T_bb =
-// ceil(L_bb / SK) * J, their inclusive scan `incl` and the total S. (More
-// batches take the looped scans of locate.)
-struct Lens64 {
-  int L;         // this lane's batch length (0 past B)
-  int64_t t;     // its stage count
-  int64_t incl;  // stage counts of batches <= this lane's, summed
+// The stage counts T_b = ceil(L_b / SK) * J of all batches, summed: lane l holds
+// those of its `per` batches [l per, (l + 1) per), so one pass of independent
+// loads, one scan and, past 64 batches, one look into one lane's share find
+// any stage's batch. (64 batches after another, a scan each and once more for
+// the total, took 30 us of every wave at 4096 batches.)
+struct BatchScan {
+  int per;       // batches per lane
+  int L;         // per == 1: this lane's batch length (0 past B)
+  int64_t t;     // stages of this lane's batches
+  int64_t incl;  // stages up to and with them
   int64_t tot;   // S, the total
 };
 template <int PG, int SK>
-__device__ inline Lens64 lens64(const DecodeParams& p, int J) {
+__device__ inline BatchScan batch_scan(const DecodeParams& p, int J) {
   const int lane = threadIdx.x & 63;
-  Lens64 r;
-  r.L = lane < p.B ? len_lane<PG>(p, lane) : 0;
-  r.t = (int64_t)((r.L + SK - 1) / SK) * J;
-  r.incl = r.t;
+  BatchScan r;
+  r.per = (p.B + 63) >> 6;
+  if (r.per == 1) {
+    r.L = lane < p.B ? len_lane<PG>(p, lane) : 0;
+    r.t = (r.L + SK - 1) / SK;
+  } else {
+    constexpr int NB = 8;  // loads in flight
+    r.L = 0;
+    r.t = 0;
+    for (int i = 0; i < r.per; i += NB) {
+      int L[NB];
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int64_t y = __shfl_up(r.incl, o);
-    if (lane >= o) r.incl += y;
+      for (int u = 0; u < NB; ++u) {
+        const int b = lane * r.per + i + u;
+        L[u] = i + u < r.per && b < p.B ? len_lane<PG>(p, b) : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < NB; ++u) r.t += (L[u] + SK - 1) / SK;
+    }
   }
-  r.tot = uni64(__shfl(r.incl, 63));
+  r.t *= J;
+  r.incl = scan64(r.t);
+  r.tot = readlane64(r.incl, 63);
   return r;
 }
 
-// The partition of all batches' stages: one length for all (PG == 0), the host
-// divided; otherwise a scan of the lengths.
+// The cursor of stage s < S of the list.
 template <int PG, int SK>
-__device__ inline Partition partition(const DecodeParams& p, int J, int W) {
-  if constexpr (PG == 0) {
-    return Partition(p.part_q, p.part_rem);
-  } else {
-    Cursor unused;
-    return Partition(locate<PG, SK>(p, J, -1, &unused), W);
+__device__ inline Cursor locate(const DecodeParams& p, int J, int64_t s, const BatchScan& sc) {
+  const int lane = threadIdx.x & 63;
+  const int ln = __builtin_ctzll(__ballot(sc.incl > s));
+  int64_t before = readlane64(sc.incl - sc.t, ln);
+  int b = ln, L = __builtin_amdgcn_readlane(sc.L, ln);
+  if (sc.per > 1) {
+    for (int i = 0; i < sc.per; i += 64) {
+      const int bb = ln * sc.per + i + lane;
+      const int Lb = i + lane < sc.per && bb < p.B ? len_lane<PG>(p, bb) : 0;
+      const int64_t t = (int64_t)((Lb + SK - 1) / SK) * J, incl = scan64(t);
+      const uint64_t hit = __ballot(before + incl > s);
+      if (hit != 0) {
+        const int in = __builtin_ctzll(hit);
+        before += readlane64(incl - t, in);
+        L = __builtin_amdgcn_readlane(Lb, in);
+        b = ln * sc.per + i + in;
+        break;
+      }
+      before += readlane64(incl, 63);
+    }
   }
+  const int nst = (L + SK - 1) / SK;
+  int64_t st;
+  const int j = (int)div_pos(uni64(s - before), nst, &st);
+  return Cursor{uni(b), uni(j), uni((int)st), uni(nst), uni(L)};
+}
+
+// The stages of batches before b (wave-uniform).
+template <int PG, int SK>
+__device__ inline int64_t stages_before(const DecodeParams& p, int J, int b, const BatchScan& sc) {
+  const int lane = threadIdx.x & 63;
+  const int ln = sc.per == 1 ? b : (int)((uint32_t)b / (uint32_t)sc.per);
+  int64_t before = readlane64(sc.incl - sc.t, ln);
+  if (sc.per > 1) {
+    int64_t t = 0;  // of this lane's share of lane ln's batches below b
+    for (int bb = ln * sc.per + lane; bb < b; bb += 64) t += (len_lane<PG>(p, bb) + SK - 1) / SK;
+    before += readlane64(scan64(t * J), 63);
+  }
+  return before;
+}
+
+// The same with one length for all batches: arithmetic.
+template <int SK>
+__device__ inline Cursor locate_uniform(const DecodeParams& p, int J, int64_t s) {
+  const int nst = (p.cache_len + SK - 1) / SK;
+  const int64_t per_b = (int64_t)nst * J;
+  int64_t r, st;
+  int b;
+  if (p.B == 1) {
+    b = 0;
+    r = s;
+  } else if ((per_b >> 31) == 0) {
+    b = (int)div_pos(s, (int)per_b, &r);
+  } else {
+    b = (int)(s / per_b);
+    r = s % per_b;
+  }
+  const int j = (int)div_pos(r, nst, &st);
+  return Cursor{uni(b), uni(j), uni((int)st), uni(nst), uni(p.cache_len)};
 }
 
 // The stages of wave w of W: their count (returned) and, if any, the cursor
-// of the first one.
+// of the first one; *part: the partition of all stages (PG == 0: the host
+// divided).
 template <int PG, int SK>
-__device__ inline int64_t wave_plan(const DecodeParams& p, int J, int W, int w, Cursor* cc) {
-  if (PG != 0 && p.B <= 64) {
-    const Lens64 ls = lens64<PG, SK>(p, J);
-    const Partition part(ls.tot, W);
-    const int64_t s0 = part.start(w);
-    const int64_t n = part.start(w + 1) - s0;
-    if (n > 0) {
-      const uint64_t hit = __ballot(ls.incl > s0);
-      const int ln = __builtin_ctzll(hit);
-      const int64_t excl = __shfl(ls.incl - ls.t, ln);
-      const int Lh = __shfl(ls.L, ln);
-      const int nst = (Lh + SK - 1) / SK;
-      int64_t st;
-      const int j = (int)div_pos(uni64(s0 - excl), nst, &st);
-      *cc = Cursor{uni(ln), uni(j), uni((int)st), uni(nst), uni(Lh)};
-    }
-    return n;
+__device__ inline int64_t wave_plan(const DecodeParams& p, int J, int W, int w, Cursor* cc, Partition* part) {
+  BatchScan sc;
+  if constexpr (PG == 0) {
+    *part = Partition(p.part_q, p.part_rem);
+  } else {
+    sc = batch_scan<PG, SK>(p, J);
+    *part = Partition(sc.tot, W);
   }
-  const Partition part = partition<PG, SK>(p, J, W);
-  const int64_t s0 = part.start(w);
-  const int64_t n = part.start(w + 1) - s0;
-  if (n > 0) locate<PG, SK>(p, J, s0, cc);
+  const int64_t s0 = part->start(w);
+  const int64_t n = part->start(w + 1) - s0;
+  if (n > 0) {
+    if constexpr (PG == 0) *cc = locate_uniform<SK>(p, J, s0);
+    else *cc = locate<PG, SK>(p, J, s0, sc);
+  }
   return n;
 }
 
@@ -442,7 +463,8 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
     cc.st = wv * per;
     n = min(per, cc.nst - cc.st);
   } else {
-    n = wave_plan<PG, SK>(p, J, W, w, &cc);
+    Partition part((int64_t)0, (int64_t)0);
+    n = wave_plan<PG, SK>(p, J, W, w, &cc, &part);
     if (n <= 0) return;
   }
 
@@ -882,15 +904,14 @@ __global__ __launch_bounds__(64 * NWV) void pf_decode_stream_kernel(DecodeParams
 // sequence of 1500 keys, 8 kv heads); 8 waves a head take 5 us. At 8-9 pieces
 // (B=16, 4096 keys): 7.5 -> 4.8 us.
 template <typename T, int D, int PG, int QR, int WPB, bool FINE>
-__global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_combine_kernel(DecodeParams p) {
+__global__ __launch_bounds__(64 * WPB) void pf_decode_stream_combine_kernel(DecodeParams p) {
   constexpr int SK = StreamGeo<T, D, FINE>::SK;
   constexpr int PER = D / 64;  // columns per lane
   constexpr int NB = 8;        // pieces in flight
   typedef float vp __attribute__((ext_vector_type(PER)));
   const int lane = threadIdx.x & 63;
   const int wv = uni((int)(threadIdx.x >> 6));
-  const int bh = WPB == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
-  if (WPB == 1 && bh >= p.B * p.Hq) return;
+  const int bh = blockIdx.x;
   const int b = p.B == 1 ? 0 : bh / p.Hq, hq = bh - b * p.Hq;
   const int g = p.g;
   const int n_hc = (g + 15) >> 4;
@@ -903,31 +924,19 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
   int64_t before = 0;     // stages of batches < b
   int L;
   if constexpr (PG == 0) {
-    part = partition<PG, SK>(p, J, W);
+    part = Partition(p.part_q, p.part_rem);
     L = p.cache_len;
     before = (int64_t)b * ((L + SK - 1) / SK) * J;
-  } else if (p.B <= 64) {
-    const Lens64 ls = lens64<PG, SK>(p, J);
-    part = Partition(ls.tot, W);
-    before = uni64(__shfl(ls.incl - ls.t, b));
-    L = __builtin_amdgcn_readfirstlane(__shfl(ls.L, b));
   } else {
-    part = partition<PG, SK>(p, J, W);
-    for (int b0 = 0; b0 < b; b0 += 64) {
-      const int bb = b0 + lane;
-      const int Lb = bb < b ? len_lane<PG>(p, bb) : 0;
-      int64_t t = (int64_t)((Lb + SK - 1) / SK) * J;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
-      before += t;
-    }
-    before = uni64(before);
-    L = len_lane<PG>(p, b);
+    const BatchScan sc = batch_scan<PG, SK>(p, J);
+    part = Partition(sc.tot, W);
+    before = stages_before<PG, SK>(p, J, uni(b), sc);
+    L = seq_len<PG>(p, uni(b));
   }
   const int nst = (L + SK - 1) / SK;
   T* out = static_cast<T*>(p.o) + (int64_t)bh * D + PER * lane;
   if (nst == 0) {
-    if (WPB == 1 || wv == 0) {
+    if (wv == 0) {
 #pragma unroll
       for (int e = 0; e < PER; ++e) out[e] = Elem<T>::from_f32(0.f);
     }
@@ -941,11 +950,11 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
   const bool late = part.start(wa) < s0;
   const int64_t seq = (int64_t)b * J + kvh * n_hc + hc;
   const int np = wb - wa + 1;
-  const int per = WPB == 1 ? np : (np + WPB - 1) / WPB;
-  const int i_end = WPB == 1 ? np : min(np, (wv + 1) * per);
+  const int per = (np + WPB - 1) / WPB;
+  const int i_end = min(np, (wv + 1) * per);
   float M = kNegInf, lsum = 0.f;  // lsum: per lane until the end
   vp o = (vp)(0.f);
-  for (int i0 = WPB == 1 ? 0 : wv * per; i0 < i_end; i0 += 64) {
+  for (int i0 = wv * per; i0 < i_end; i0 += 64) {
     const int cnt = min(64, i_end - i0);
     f32x2 ml = {kNegInf, 0.f};
     if (lane < cnt) {
@@ -981,51 +990,155 @@ __global__ __launch_bounds__(WPB == 1 ? 256 : 64 * WPB) void pf_decode_stream_co
   }
 #pragma unroll
   for (int s = 1; s < 64; s <<= 1) lsum += __shfl_xor(lsum, s);
-  if constexpr (WPB > 1) {
-    __shared__ float sm[WPB][2];
-    __shared__ vp so[WPB][64];
-    if (lane == 0) {
-      sm[wv][0] = M;
-      sm[wv][1] = lsum;
-    }
-    so[wv][lane] = o;
-    __syncthreads();
-    if (wv != 0) return;
-    M = kNegInf;
+  __shared__ float sm[WPB][2];
+  __shared__ vp so[WPB][64];
+  if (lane == 0) {
+    sm[wv][0] = M;
+    sm[wv][1] = lsum;
+  }
+  so[wv][lane] = o;
+  __syncthreads();
+  if (wv != 0) return;
+  M = kNegInf;
 #pragma unroll
-    for (int i = 0; i < WPB; ++i) M = fmaxf(M, sm[i][0]);
-    const float Mu = (M == kNegInf) ? 0.f : M;
-    lsum = 0.f;
-    o = (vp)(0.f);
+  for (int i = 0; i < WPB; ++i) M = fmaxf(M, sm[i][0]);
+  const float Mu = (M == kNegInf) ? 0.f : M;
+  lsum = 0.f;
+  o = (vp)(0.f);
 #pragma unroll
-    for (int i = 0; i < WPB; ++i) {
-      if (i * per >= np) break;  // a wave without pieces holds nothing
-      const float wt = exp2f(sm[i][0] - Mu);
-      lsum += sm[i][1] * wt;
-      o += so[i][lane] * wt;
-    }
+  for (int i = 0; i < WPB; ++i) {
+    if (i * per >= np) break;  // a wave without pieces holds nothing
+    const float wt = exp2f(sm[i][0] - Mu);
+    lsum += sm[i][1] * wt;
+    o += so[i][lane] * wt;
   }
   const float inv = (lsum == 0.f) ? 0.f : 1.f / lsum;
 #pragma unroll
   for (int e = 0; e < PER; ++e) out[e] = Elem<T>::from_f32(o[e] * inv);
 }
 
-// Waves per (b, h) of the combine: its pieces, about n_waves / sequences (and
-// at most one per stage), decide. Few pieces: a wave each, four (b, h) to a
-// workgroup; more: 4 or 8 waves share them.
+// The same for sequences in few pieces: a workgroup per wave boundary, that is
+// per place where a sequence can be cut at all. The first boundary inside a
+// sequence takes it: one wave finds it in the work list for all four, and the
+// workgroup's threads take 4 columns of a head each. The last workgroups write
+// the zeros of batches without a valid key. Bound by the search's and the
+// pieces' latency. A wave per (b, h), each with a search of its own, mostly to
+// find that its sequence is whole, took 30 us at 19200 heads and, with the
+// batch-by-batch search, 855 us at 65536 (bf16 head_dim 64, 300 x 64 and
+// 4096 x 16 heads of up to 128 and 64 keys; now 7 and 24), more than the
+// attention itself; at 2048 and 4096 heads of head_dim 128 5.0 -> 4.9 and
+// 7.5 -> 4.9 us.
+template <typename T, int D, int PG, int QR, bool FINE>
+__global__ __launch_bounds__(256) void pf_decode_stream_cut_kernel(DecodeParams p) {
+  constexpr int SK = StreamGeo<T, D, FINE>::SK;
+  const int lane = threadIdx.x & 63;
+  const int wv = uni((int)(threadIdx.x >> 6));
+  const int g = p.g;
+  const int n_hc = (g + 15) >> 4;
+  const int J = p.Hkv * n_hc;
+  const int W = p.n_waves;
+  const int w = blockIdx.x + 1;
+  if (PG != 0 && w >= W) {
+    const int b = (w - W) * 4 + wv;
+    if (b >= p.B || seq_len<PG>(p, b) > 0) return;
+    typedef T v4 __attribute__((ext_vector_type(4)));
+    v4* out = reinterpret_cast<v4*>(static_cast<T*>(p.o) + (int64_t)b * p.Hq * D);
+    const int64_t n = (int64_t)p.Hq * (D / 4);
+    for (int64_t i = lane; i < n; i += 64) out[i] = (v4)(Elem<T>::from_f32(0.f));
+    return;
+  }
+  __shared__ int found[4];  // pieces, batch, sequence within it, late
+  if (wv == 0) {
+    Cursor c{0, 0, 0, 0, 0};
+    Partition part((int64_t)0, (int64_t)0);
+    int np = 0;
+    bool late = false;
+    if (wave_plan<PG, SK>(p, J, W, w, &c, &part) > 0 && c.st > 0) {
+      const int64_t s0 = part.start(w) - c.st, before = part.start(w - 1);
+      late = before < s0;
+      if (before <= s0) np = part.wave_of(s0 + c.nst - 1) - w + 2;
+    }
+    if (lane == 0) {
+      found[0] = np;
+      found[1] = c.b;
+      found[2] = c.j;
+      found[3] = late;
+    }
+  }
+  __syncthreads();
+  const int np = uni(found[0]), b = uni(found[1]), j = uni(found[2]);
+  const bool late = uni(found[3]) != 0;
+  if (np == 0) return;
+  const int kvh = j / n_hc, hc = j - kvh * n_hc;
+  const int nq = min(16, g - 16 * hc);
+  const int64_t seq = (int64_t)b * J + j;
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  T* out = static_cast<T*>(p.o) + ((int64_t)b * p.Hq + (int64_t)kvh * g + hc * 16) * D;
+  constexpr int NB = 8;  // pieces in flight
+  for (int i = threadIdx.x; i < nq * (D / 4); i += 256) {
+    const int qi = i / (D / 4), d0 = 4 * (i % (D / 4));
+    float M = kNegInf, l = 0.f;
+    f32x4 o = (f32x4)(0.f);
+    for (int c0 = 0; c0 < np; c0 += NB) {
+      float ls[NB];
+      f32x2 ml[NB];
+      f32x4 v[NB];
+      float Mn = M;
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        ml[c] = (f32x2){kNegInf, 0.f};
+        v[c] = (f32x4)(0.f);
+        if (c0 + c < np) {
+          const int64_t row = piece_slot(p, J, w - 1 + c0 + c, seq, c0 + c == 0 && late) * QR + qi;
+          ml[c] = *reinterpret_cast<const f32x2*>(p.part_ml + row * 2);
+          v[c] = *reinterpret_cast<const f32x4*>(p.part_o + row * D + d0);
+        }
+        Mn = fmaxf(Mn, ml[c][0]);
+      }
+      const float Mu = (Mn == kNegInf) ? 0.f : Mn;
+      const float back = exp2f(M - Mu);
+      o *= back;
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        const float wt = exp2f(ml[c][0] - Mu);
+        ls[c] = ml[c][1] * wt;
+        o += v[c] * wt;
+      }
+      {
+        // in the order of pf_decode_stream_combine_kernel's lanes, unfused: up
+        // to NB pieces give its bits
+#pragma clang fp contract(off)
+        l = l * back + (((ls[0] + ls[1]) + (ls[2] + ls[3])) + ((ls[4] + ls[5]) + (ls[6] + ls[7])));
+      }
+      M = Mn;
+    }
+    const float inv = (l == 0.f) ? 0.f : 1.f / l;
+    v4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = Elem<T>::from_f32(o[e] * inv);
+    *reinterpret_cast<v4*>(out + qi * D + d0) = y;
+  }
+}
+
+// The merge's form: the pieces of a sequence, about n_waves / sequences (and at
+// most one per stage), decide. Few: a workgroup per wave boundary; more than 6,
+// where the sequences are at most a sixth of the waves: 4 or 8 waves share the
+// pieces of each (b, h).
 template <typename T, int D, int PG, int QR, bool FINE>
 hipError_t launch_combine(const DecodeParams& p, hipStream_t st) {
   const int64_t n_bh = (int64_t)p.B * p.Hq;
   const int64_t seqs = (int64_t)p.B * p.Hkv * ((p.Hq / p.Hkv + 15) / 16);
   const int64_t len = PG <= 1 ? p.cache_len : (int64_t)p.pages_per_seq * p.page_size;
   const int64_t pieces = std::min((int64_t)p.n_waves / seqs, len / StreamGeo<T, D, FINE>::SK) + 1;
-  if (pieces > 32)
+  if (pieces > 32) {
     hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 8, FINE>), dim3((unsigned)n_bh), dim3(512), 0, st, p);
-  else if (pieces > 6)
+  } else if (pieces > 6) {
     hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 4, FINE>), dim3((unsigned)n_bh), dim3(256), 0, st, p);
-  else
-    hipLaunchKernelGGL((pf_decode_stream_combine_kernel<T, D, PG, QR, 1, FINE>), dim3((unsigned)((n_bh + 3) / 4)),
-                       dim3(256), 0, st, p);
+  } else {
+    const int64_t n = p.n_waves - 1 + (PG == 0 ? 0 : (p.B + 3) / 4);  // a wave per batch for the zeros
+    if (n > 0)
+      hipLaunchKernelGGL((pf_decode_stream_cut_kernel<T, D, PG, QR, FINE>), dim3((unsigned)n), dim3(256), 0, st, p);
+  }
   return hipGetLastError();
 }
 
