@@ -285,10 +285,11 @@ __device__ inline int64_t scan64(int64_t x) {
 // The stage counts T_b = ceil(L_b / SK) * J of all batches, summed: lane l holds
 // those of its `per` batches [l per, (l + 1) per), so one pass of independent
 // loads, one scan and, past 64 batches, one look into one lane's share find
-// any stage's batch. (64 batches after another, a scan each and once more for
-// the total, took 30 us of every wave at 4096 batches.)
+// any stage's batch. The lanes' loads lie in 64 cache lines, so a paged call
+// takes 4 lengths with each. (64 batches after another, a scan each and once
+// more for the total, took 30 us of every wave at 4096 batches.)
 struct BatchScan {
-  int per;       // batches per lane
+  int per;       // batches per lane: 1, or a multiple of 4
   int L;         // per == 1: this lane's batch length (0 past B)
   int64_t t;     // stages of this lane's batches
   int64_t incl;  // stages up to and with them
@@ -298,24 +299,39 @@ template <int PG, int SK>
 __device__ inline BatchScan batch_scan(const DecodeParams& p, int J) {
   const int lane = threadIdx.x & 63;
   BatchScan r;
-  r.per = (p.B + 63) >> 6;
-  if (r.per == 1) {
+  r.per = 1;
+  if (p.B <= 64) {
     r.L = lane < p.B ? len_lane<PG>(p, lane) : 0;
     r.t = (r.L + SK - 1) / SK;
   } else {
-    constexpr int NB = 8;  // loads in flight
+    typedef int i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int NB = 16;  // lengths in flight
+    r.per = (((p.B + 63) >> 6) + 3) & ~3;
     r.L = 0;
     r.t = 0;
-    for (int i = 0; i < r.per; i += NB) {
+    const int b0 = lane * r.per, b1 = min(b0 + r.per, p.B);
+    int b = b0;
+    for (; b + NB <= b1; b += NB) {
       int L[NB];
+      if constexpr (PG > 1) {
 #pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        const int b = lane * r.per + i + u;
-        L[u] = i + u < r.per && b < p.B ? len_lane<PG>(p, b) : 0;
+        for (int u = 0; u < NB / 4; ++u) {
+          const i32x4u x = *reinterpret_cast<const i32x4u*>(p.context_lens + b + 4 * u);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) L[4 * u + e] = min(max(x[e], 0), p.pages_per_seq * p.page_size);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) L[u] = len_lane<PG>(p, b + u);
       }
 #pragma unroll
       for (int u = 0; u < NB; ++u) r.t += (L[u] + SK - 1) / SK;
     }
+    int L[NB];  // the share's rest
+#pragma unroll
+    for (int u = 0; u < NB; ++u) L[u] = b + u < b1 ? len_lane<PG>(p, b + u) : 0;
+#pragma unroll
+    for (int u = 0; u < NB; ++u) r.t += (L[u] + SK - 1) / SK;
   }
   r.t *= J;
   r.incl = scan64(r.t);
@@ -1025,9 +1041,9 @@ __global__ __launch_bounds__(64 * WPB) void pf_decode_stream_combine_kernel(Deco
 // pieces' latency. A wave per (b, h), each with a search of its own, mostly to
 // find that its sequence is whole, took 30 us at 19200 heads and, with the
 // batch-by-batch search, 855 us at 65536 (bf16 head_dim 64, 300 x 64 and
-// 4096 x 16 heads of up to 128 and 64 keys; now 7 and 24), more than the
+// 4096 x 16 heads of up to 128 and 64 keys; now 8 and 10), more than the
 // attention itself; at 2048 and 4096 heads of head_dim 128 5.0 -> 4.9 and
-// 7.5 -> 4.9 us.
+// 7.5 -> 5.9 us.
 template <typename T, int D, int PG, int QR, bool FINE>
 __global__ __launch_bounds__(256) void pf_decode_stream_cut_kernel(DecodeParams p) {
   constexpr int SK = StreamGeo<T, D, FINE>::SK;
