@@ -283,8 +283,9 @@ void bind_fwd_split(const pf_attn_fwd_args* a, pf::FwdParams* p, void* ws) {
   p->part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + align_ws(prow * a->head_dim * 4));
 }
 
-// Minimum items for a dynamic tail: two per resident workgroup slot of a
-// 256-CU MI355X (the 16-bit forward and dQ run two workgroups per CU).
+// Minimum items for a dynamic tail: four per CU of a 256-CU MI355X, two per
+// resident workgroup where two are resident (the 16-bit forward and dQ; at
+// head_dim 64 the forward has three, so 1.33).
 constexpr int kTwoPerCu = 2 * 2 * 256;
 
 }  // namespace
@@ -609,7 +610,7 @@ static int stream_setup(pf::DecodeParams* p, int dtype, int64_t max_len) {
   const int sk = p->D * (f32 ? 4 : 2) == 512 || p->fine ? 16 : 32;  // keys per stage
   const int unit = f32 ? sk : 32;
   const int64_t runs = seqs * ((max_len + unit - 1) / unit);
-  const int grid = stream_grid(dtype, p->D, group, p->fine != 0);
+  const int grid = p->full_waves = stream_grid(dtype, p->D, group, p->fine != 0);
   p->n_waves = grid > runs ? (int)(runs > 1 ? runs : 1) : grid;
   p->n_split = 0;
   p->chunk = 0;
@@ -639,7 +640,8 @@ static bool stream_only(int32_t head_dim, int32_t dtype) { return head_dim == 12
 // at least a batch's heads, for the generic kernel.
 static int64_t stream_room(const pf::DecodeParams& p, int dtype) {
   const int group = p.Hq / p.Hkv;
-  return std::max((int64_t)2 * stream_grid(dtype, p.D, group, false) * pf::decode_stream_qrows(group), (int64_t)p.Hq);
+  const int grid = p.full_waves > 0 ? p.full_waves : stream_grid(dtype, p.D, group, false);
+  return std::max((int64_t)2 * grid * pf::decode_stream_qrows(group), (int64_t)p.Hq);
 }
 
 // The generic kernel's chunks of up to max_len keys. room > 0: no more partials
@@ -732,12 +734,10 @@ static size_t decode_ws_most(const pf::DecodeParams& p, int dtype, bool streams,
 }
 
 // The bytes that a launch insists on: what it uses; the 16-bit head_dim 128
-// forms the full size that their query answers (or more, where another thread
-// has just lowered decode_waves).
+// forms the full size that their query answers.
 static size_t decode_ws_bytes(const pf::DecodeParams& p, int dtype, bool streams) {
-  const size_t used = partial_bytes(decode_slots(p), p.D);
-  if (!streams || !stream_only(p.dr, dtype)) return used;
-  return std::max(used, decode_ws_most(p, dtype, true, 0));
+  if (streams && stream_only(p.dr, dtype)) return decode_ws_most(p, dtype, true, 0);
+  return partial_bytes(decode_slots(p), p.D);
 }
 
 static int bind_workspace(pf::DecodeParams* p, int dtype, bool streams, void* ws, size_t bytes) {

@@ -288,6 +288,7 @@ struct DecodeParams {
   int fine;           // 16-key stages (float32 head_dim 64)
   int fixed_grid;     // n_waves was set by hand (tuning): keep the persistent grid
   int slice;          // generic kernel: batches per launch
+  int full_waves;     // streaming kernel: the waves that are resident at once (host only)
   int n_waves;        // streaming kernel: persistent grid (one wave per workgroup); 0: generic kernel
   // Fused decode step (streaming kernel, positions != null): the new token of
   // batch b is at pos = positions[b * pos_stride]; its k (rotated with table
