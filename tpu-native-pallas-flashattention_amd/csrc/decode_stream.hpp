@@ -947,7 +947,7 @@ __global__ __launch_bounds__(64 * WPB) void pf_decode_stream_combine_kernel(Deco
     const BatchScan sc = batch_scan<PG, SK>(p, J);
     part = Partition(sc.tot, W);
     before = stages_before<PG, SK>(p, J, uni(b), sc);
-    L = seq_len<PG>(p, uni(b));
+    L = sc.per == 1 ? __builtin_amdgcn_readlane(sc.L, uni(b)) : seq_len<PG>(p, uni(b));
   }
   const int nst = (L + SK - 1) / SK;
   T* out = static_cast<T*>(p.o) + (int64_t)bh * D + PER * lane;
