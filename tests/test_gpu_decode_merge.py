@@ -81,9 +81,9 @@ def test_step_over_many_sequences(w, Hq, Hkv):
 
 
 def test_the_merge_of_many_heads_is_a_small_part():
-    """4096 x 16 heads of up to 64 keys, two fifths of the pool's 268 MB: less than
-    6 copies of its K half (about 50 us each). The call takes about 75 us; with a
-    search per head in the merge it took 950."""
+    """4096 x 16 heads of 8-64 keys, a little over half of the pool's 268 MB: less
+    than 6 copies of its K half (about 50 us each). The kernels take 47 us; with
+    a search per head in the merge they took 945."""
     note("decode merge: time")
     B, Hq, Hkv, page, D = 4096, 16, 4, 64, 64
     gen = torch.Generator("cuda").manual_seed(1)
